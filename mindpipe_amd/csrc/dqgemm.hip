@@ -16,7 +16,7 @@
 // fraction of an output ulp: the fake-rule MoE expert chain (a 1-ulp change of a gate / up
 // value flips codes of the coarse per-token requant that follows), the bf16 fake-rule W8A8
 // linear and the bf16 W4A16 linear (bf16 rounding of each dequantised weight is ~2^-9).
-#include "dq_gemm.h"
+#include "dq_wide.h"
 
 namespace {
 
@@ -418,6 +418,7 @@ int mp_launch_dq_gemm(const mp_dq_args &p, int epi, hipStream_t stream) {
   // 32-bit descriptor offsets over A and 32-bit tile arithmetic
   if (p.rows * p.k * (p.a_fmt == MP_DQ_DT ? 2 : 1) >= (int64_t(1) << 31) || p.k > (1 << 20)) return MP_ERR_SHAPE;
   if (p.k % kDBK == 0 && (!mp_aligned(p.a, 16) || !mp_aligned(p.b, 16))) return MP_ERR_ALIGN;  // tiled loads
+  if (mp_dq_wide_takes(p, epi)) return mp_launch_dq_wide(p, epi, stream);
   const bool a8 = p.a_fmt == MP_DQ_I8ROW, b8 = p.b_fmt == MP_DQ_I8ROW;
   if (u4 && a8) return MP_ERR_ARG;  // packed weights multiply plain activations only
   if (p.dt == MP_F16) {

@@ -2,7 +2,7 @@
 // with the per-token int8 quant, GMM1 + SwiGLU + requant, GMM2, and the
 // weighted un-permute.  The two grouped GEMMs use the tiled int8 MFMA kernel
 // of w8a8.hip with a grouped row schedule.
-#include "dq_gemm.h"
+#include "dq_wide.h"
 
 #include <mutex>
 
@@ -248,8 +248,9 @@ __global__ __launch_bounds__(256) void moe_requant_kernel(const float *__restric
 //                 one rounding to out_dtype.
 //   FAKE = true : the reference's index_add_ in out_dtype r: over the assignments in
 //                 ascending expert order (= ascending routed row), out = r(out + r(r(y) * w)).
-template <bool FAKE, bool VEC>
-__global__ __launch_bounds__(256) void moe_combine_kernel(const float *__restrict__ y,
+// YDT: the dtype of y (a 16-bit y holds r(y) already: the same bits, half the traffic).
+template <bool FAKE, bool VEC, int YDT>
+__global__ __launch_bounds__(256) void moe_combine_kernel(const void *__restrict__ y_,
                                                          const int32_t *__restrict__ row_of_slot,
                                                          const float *__restrict__ w, int64_t t_count, int top_k,
                                                          int64_t h, void *__restrict__ out, int out_dtype) {
@@ -284,14 +285,22 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(const float *__restric
     }
     const float wj = w[t * top_k + slot];
     float v[NC];
-    if constexpr (VEC) {
-      const float4 y4 = *reinterpret_cast<const float4 *>(y + static_cast<int64_t>(r) * h + c);
+    const int64_t at = static_cast<int64_t>(r) * h + c;
+    if constexpr (VEC && YDT == MP_F32) {
+      const float4 y4 = *reinterpret_cast<const float4 *>(static_cast<const float *>(y_) + at);
       v[0] = y4.x;
       v[1] = y4.y;
       v[2] = y4.z;
       v[3] = y4.w;
+    } else if constexpr (VEC) {
+      const uint2 y2 = *reinterpret_cast<const uint2 *>(static_cast<const uint16_t *>(y_) + at);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const uint16_t b = static_cast<uint16_t>((i < 2 ? y2.x : y2.y) >> (16 * (i & 1)));
+        v[i] = YDT == MP_F16 ? mp_h2f(b) : mp_bf2f(b);
+      }
     } else {
-      v[0] = y[static_cast<int64_t>(r) * h + c];
+      v[0] = mp_load_as_f32(y_, at, YDT);
     }
 #pragma unroll
     for (int i = 0; i < NC; ++i) {
@@ -539,7 +548,7 @@ extern "C" int mp_moe_unpermute_combine(const float *y, const int32_t *row_of_sl
   const bool vec = h % 4 == 0 && mp_aligned(y, 16) && mp_aligned(out, out_dtype == MP_F32 ? 16 : 8);
   const dim3 g(static_cast<unsigned>(mp_cdiv(vec ? t * (h / 4) : t * h, 256)));
 #define MP_CB(FAKE_, VEC_) \
-  hipLaunchKernelGGL((moe_combine_kernel<FAKE_, VEC_>), g, dim3(256), 0, st, y, row_of_slot, topk_w, t, top_k, h, out, \
+  hipLaunchKernelGGL((moe_combine_kernel<FAKE_, VEC_, MP_F32>), g, dim3(256), 0, st, y, row_of_slot, topk_w, t, top_k, h, out, \
                      out_dtype)
   if (scale_rule == MP_SCALE_FAKE) {
     if (vec) MP_CB(true, true);
@@ -595,6 +604,96 @@ extern "C" int mp_i8_gemm_swiglu_requant_noalloc(const int8_t *routed, const flo
 }
 
 // ---------------------------------------------------------------- misc
+// The fake-rule chain with its tensors in the dtype the reference module holds them in: routed
+// fake-quantized rows, h, h fake-quantized in place, and the down output, each 16 bits per value instead of
+// codes plus an fp32 buffer.  The values are those of the four separate entry points: every one is rounded to
+// the dtype there too, before its next use.
+static size_t mp_moe_fake_part(size_t &at, size_t bytes) {
+  const size_t o = at;
+  at += (bytes + 255) & ~static_cast<size_t>(255);
+  return o;
+}
+struct mp_moe_fake_layout {
+  size_t slots, offsets, a16, h16, y, total;
+  mp_moe_fake_layout(int64_t t, int64_t h, int64_t inter, int top_k, int n_experts) {
+    const size_t rows = static_cast<size_t>(t) * static_cast<size_t>(top_k);
+    size_t at = 0;
+    slots = mp_moe_fake_part(at, rows * sizeof(int32_t));
+    offsets = mp_moe_fake_part(at, (static_cast<size_t>(n_experts) + 1) * sizeof(int64_t));
+    a16 = mp_moe_fake_part(at, rows * static_cast<size_t>(h) * 2);
+    h16 = mp_moe_fake_part(at, rows * static_cast<size_t>(inter) * 2);
+    y = mp_moe_fake_part(at, rows * static_cast<size_t>(h) * 2);
+    total = at;
+  }
+};
+
+extern "C" size_t mp_moe_fake_workspace_bytes(int64_t t, int64_t h, int64_t inter, int top_k, int n_experts) {
+  if (t <= 0 || h <= 0 || inter <= 0 || top_k <= 0 || n_experts <= 0) return 0;
+  return mp_moe_fake_layout(t, h, inter, top_k, n_experts).total;
+}
+
+extern "C" int mp_moe_fake_forward(const void *x, int x_dtype, int64_t t, int64_t h, const int32_t *topk_ids,
+                                   const float *topk_w, int top_k, int n_experts, const int8_t *w13, const float *s13,
+                                   const int8_t *w2, const float *s2, int64_t inter, void *out, int out_dtype,
+                                   void *workspace, size_t workspace_bytes, mp_stream_t stream) {
+  if (!x || !topk_ids || !topk_w || !w13 || !s13 || !w2 || !s2 || !out) return MP_ERR_ARG;
+  if (x_dtype != MP_F16 && x_dtype != MP_BF16) return MP_ERR_DTYPE;
+  if (out_dtype != MP_F16 && out_dtype != MP_BF16) return MP_ERR_DTYPE;
+  if (t < 0 || h <= 0 || inter <= 0 || top_k <= 0 || top_k > 64 || n_experts <= 0 || n_experts > kMaxExperts) return MP_ERR_SHAPE;
+  if (t * top_k > INT32_MAX) return MP_ERR_SHAPE;
+  if (t == 0) return MP_OK;
+  const mp_moe_fake_layout l(t, h, inter, top_k, n_experts);
+  if (!workspace || workspace_bytes < l.total) return MP_ERR_WORKSPACE;
+  if (!mp_aligned(workspace, 16) || !mp_aligned(out, 8)) return MP_ERR_ALIGN;
+  char *ws = static_cast<char *>(workspace);
+  auto *slots = reinterpret_cast<int32_t *>(ws + l.slots);
+  auto *offsets = reinterpret_cast<int64_t *>(ws + l.offsets);
+  const int64_t rows = t * top_k;
+  mp_dq_args d{};
+  d.dt = x_dtype;
+  d.a_fmt = MP_DQ_DT;
+  d.b_fmt = MP_DQ_I8ROW;
+  d.offsets = offsets;
+  d.n_experts = n_experts;
+  d.rows = rows;
+  mp_dq_args d1 = d, d2 = d;
+  d1.a = ws + l.a16;
+  d1.b = w13;
+  d1.b_scale = s13;
+  d1.y = ws + l.h16;
+  d1.out_dtype = x_dtype;
+  d1.ldy = inter;
+  d1.n = inter;
+  d1.k = h;
+  d2.a = ws + l.h16;
+  d2.b = w2;
+  d2.b_scale = s2;
+  d2.y = ws + l.y;
+  d2.out_dtype = out_dtype;
+  d2.ldy = h;
+  d2.n = h;
+  d2.k = inter;
+  if (!mp_dq_wide_takes(d1, MP_EPI_SWIGLU) || !mp_dq_wide_takes(d2, MP_EPI_DENSE) || inter % 64) return MP_ERR_SHAPE;
+  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  hipLaunchKernelGGL(moe_route_kernel, dim3(1), dim3(64 * kRouteWaves), 0, s, topk_ids, rows, n_experts, offsets, slots,
+                     static_cast<int32_t *>(nullptr));
+  MP_CHECK_LAUNCH();
+  int rc = mp_launch_fake_values(x, x_dtype, rows, h, slots, top_k, ws + l.a16, s);
+  if (rc == MP_OK) rc = mp_launch_dq_wide(d1, MP_EPI_SWIGLU, s);
+  if (rc == MP_OK) rc = mp_launch_fake_values(ws + l.h16, x_dtype, rows, inter, nullptr, 1, ws + l.h16, s);
+  if (rc == MP_OK) rc = mp_launch_dq_wide(d2, MP_EPI_DENSE, s);
+  if (rc != MP_OK) return rc;
+  const dim3 g(static_cast<unsigned>(mp_cdiv(t * (h / 4), 256)));
+#define MP_FC(DT_)                                                                                                  \
+  hipLaunchKernelGGL((moe_combine_kernel<true, true, DT_>), g, dim3(256), 0, s, ws + l.y, slots, topk_w, t, top_k, h, \
+                     out, out_dtype)
+  if (out_dtype == MP_F16) MP_FC(MP_F16);
+  else MP_FC(MP_BF16);
+#undef MP_FC
+  MP_CHECK_LAUNCH();
+  return MP_OK;
+}
+
 extern "C" const char *mp_strerror(int status) {
   switch (status) {
     case MP_OK: return "ok";

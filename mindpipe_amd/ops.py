@@ -371,6 +371,40 @@ def _(qx, s_tok, w, s_ch, bias, act_dtype):
     return qx.new_empty((*qx.shape[:-1], w.shape[0]), dtype=act_dtype)
 
 
+# in a namespace of its own: torch.ops.mindpipe_amd holds the reference's operator contracts
+@torch.library.custom_op("mindpipe_amd_fake::w8a8_linear", mutates_args=())
+def w8a8_linear_fake(x: torch.Tensor, w: torch.Tensor, s_ch: torch.Tensor,
+                     bias: Optional[torch.Tensor]) -> torch.Tensor:
+    """``F.linear(fake_quant(x), r(w * s_ch), bias)`` in ``x``'s dtype (fp16 / bf16): the per-token
+    fake quant of ``x [..., K]`` (``fake_quant.py:22-31``) and the linear on it in one call, without
+    codes in between; ``w8a8_gemm_fake`` is the same on codes."""
+    _need(x, "x", (torch.float16, torch.bfloat16))
+    _need(w, "w", torch.int8, 2)
+    _need(s_ch, "s_ch", torch.float32, 1)
+    k = x.shape[-1]
+    n = w.shape[0]
+    if w.shape[1] != k:
+        raise RuntimeError(f"weight {tuple(w.shape)} does not match K={k}")
+    if s_ch.numel() != n:
+        raise RuntimeError("scale sizes do not match M / N")
+    if bias is not None:
+        _need(bias, "bias", x.dtype, 1)
+    x2 = x.reshape(-1, k)
+    m = x2.shape[0]
+    y = torch.empty((*x.shape[:-1], n), dtype=x.dtype, device=x.device)
+    ws = torch.empty((m, k), dtype=x.dtype, device=x.device)
+    with _dev(x):
+        _lib.check(_lib.load().mp_w8a8_linear_fake(
+            x2.data_ptr(), _DT[x.dtype], m, k, w.data_ptr(), s_ch.data_ptr(), n, _ptr(bias), y.data_ptr(),
+            ws.data_ptr(), ws.numel() * 2, _stream()), "mp_w8a8_linear_fake")
+    return y
+
+
+@w8a8_linear_fake.register_fake
+def _(x, w, s_ch, bias):
+    return x.new_empty((*x.shape[:-1], w.shape[0]))
+
+
 # ---------------------------------------------------------------- MoE
 _RULES = {"runtime": MP_SCALE_FP32, "fake": MP_SCALE_FAKE}
 
@@ -588,6 +622,40 @@ def moe_unpermute_combine(y, row_of_slot, topk_w, out_dtype=torch.float16, rule:
     return out
 
 
+def _moe_fake_takes(x, topk_ids, topk_w, w13, s13, w2, s2, out_dtype) -> bool:
+    """Whether ``mp_moe_fake_forward`` takes the call: well-formed operands (the four entry points
+    raise for others) of the sizes and alignments it reads."""
+    dev = x.device
+    if not (x.is_cuda and x.dim() == 2 and x.is_contiguous() and topk_ids.dim() == 2 and w13.dim() == 3 and
+            w2.dim() == 3 and out_dtype in (torch.float16, torch.bfloat16)):
+        return False
+    t, h = x.shape
+    e, inter = w13.shape[0], w2.shape[2]
+    return (t > 0 and topk_ids.shape[0] == t and 0 < topk_ids.shape[1] <= 64 and topk_w.shape == topk_ids.shape and
+            w13.shape == (e, 2 * inter, h) and w2.shape == (e, h, inter) and s13.shape == (e, 2 * inter) and
+            s2.shape == (e, h) and w13.dtype == w2.dtype == torch.int8 and s13.dtype == s2.dtype == torch.float32 and
+            all(v.device == dev and v.is_contiguous() for v in (w13, w2, s13, s2)) and
+            topk_ids.device == dev and topk_w.device == dev and 0 < e <= 1024 and h % 64 == 0 and inter % 64 == 0 and
+            h <= 1 << 17 and 2 * inter * h < 1 << 31 and t * topk_ids.shape[1] < 1 << 27 and
+            w13.data_ptr() % 16 == 0 and w2.data_ptr() % 16 == 0)
+
+
+def _moe_fake(x, topk_ids, topk_w, w13, s13, w2, s2, out_dtype):
+    t, h = x.shape
+    e, inter, top_k = w13.shape[0], w2.shape[2], topk_ids.shape[1]
+    ids, tw = topk_ids.to(torch.int32).contiguous(), topk_w.to(torch.float32).contiguous()
+    out = torch.empty((t, h), dtype=out_dtype, device=x.device)
+    lib = _lib.load()
+    wsb = lib.mp_moe_fake_workspace_bytes(t, h, inter, top_k, e)
+    ws = torch.empty((wsb,), dtype=torch.uint8, device=x.device)
+    with _dev(x):
+        _lib.check(lib.mp_moe_fake_forward(
+            x.data_ptr(), _DT[x.dtype], t, h, ids.data_ptr(), tw.data_ptr(), top_k, e, w13.data_ptr(),
+            s13.data_ptr(), w2.data_ptr(), s2.data_ptr(), inter, out.data_ptr(), _DT[out_dtype], ws.data_ptr(), wsb,
+            _stream()), "mp_moe_fake_forward")
+    return out
+
+
 @torch.library.custom_op("mindpipe_amd::moe_w8a8_forward", mutates_args=())
 def moe_w8a8_forward(x: torch.Tensor, topk_ids: torch.Tensor, topk_w: torch.Tensor, w13: torch.Tensor,
                      s13: torch.Tensor, w2: torch.Tensor, s2: torch.Tensor, out_dtype: Optional[torch.dtype] = None,
@@ -605,6 +673,8 @@ def moe_w8a8_forward(x: torch.Tensor, topk_ids: torch.Tensor, topk_w: torch.Tens
     act_dtype = x.dtype if x_scale is None else out_dtype
     if rule == "fake" and act_dtype not in (torch.float16, torch.bfloat16):
         raise RuntimeError("the fake rule runs in fp16 or bf16")
+    if rule == "fake" and x_scale is None and _moe_fake_takes(x, topk_ids, topk_w, w13, s13, w2, s2, out_dtype):
+        return _moe_fake(x, topk_ids, topk_w, w13, s13, w2, s2, out_dtype)
     routed, rscale, row_of_slot, offsets = moe_permute_quant(x, topk_ids.to(torch.int32).contiguous(), e, rule,
                                                              x_scale)
     q, s = moe_gmm1_swiglu_quant(routed, rscale, w13, s13, offsets, inter, rule, act_dtype)

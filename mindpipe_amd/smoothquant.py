@@ -196,6 +196,8 @@ class SmoothQuantLinear(nn.Module):
         _require_gpu(x, "SmoothQuantLinear")
         if not self._w8a8:
             return self.output_quant(self._linear_any_width(x))
+        if self._bf16_fake(x):
+            return self.output_quant(self._linear_values(x))
         fake, q, s = self._input_codes(x)
         if self._fused_output_quant(x, fake):
             qo, so = self._output_codes(q, s, x.dtype)
@@ -209,12 +211,19 @@ class SmoothQuantLinear(nn.Module):
         q, s = ops.quant_per_token_i8(x.contiguous(), fake)
         return fake, q, s
 
+    def _bf16_fake(self, x) -> bool:
+        return self.scale_rule == "fake" and x.dtype == torch.bfloat16
+
+    def _linear_values(self, x):
+        """The bf16 fake-rule linear: bf16 keeps 8 significant bits, and the reference multiplies the
+        bf16-rounded fake values r(q * s), which the int8 product of q * s misses by ~3e-3; the
+        dequantising GEMM rounds each element as the reference does."""
+        bias = None if self.bias is None else self.bias.to(torch.bfloat16)
+        return ops.w8a8_linear_fake(x.contiguous(), self.weight, self.weight_scale, bias)
+
     def _linear(self, x, fake, q, s):
-        """The linear's output before any output quant."""
+        """The linear's output on the input's codes, before any output quant."""
         if fake and x.dtype == torch.bfloat16:
-            # bf16 keeps 8 significant bits: the reference multiplies the bf16-rounded fake values
-            # r(q * s), which the int8 product of q * s misses by ~3e-3; the dequantising GEMM
-            # rounds each element as the reference does
             bias = None if self.bias is None else self.bias.to(torch.bfloat16)
             return ops.w8a8_gemm_fake(q, s.float().contiguous(), self.weight, self.weight_scale, bias, x.dtype)
         return ops.w8a8_gemm(q, s.float().contiguous(), self.weight, self.weight_scale, self.bias, x.dtype)
@@ -244,6 +253,8 @@ class SmoothQuantLinear(nn.Module):
         if not self._w8a8:
             y = self._linear_any_width(x)
             return _row_codes(y.reshape(-1, self.out_features).contiguous(), self.activation_bits)
+        if self._bf16_fake(x):
+            return ops.quant_per_token_i8(self._linear_values(x).contiguous(), True)
         fake, q, s = self._input_codes(x)
         if self._fused_output_quant(x, fake):
             return self._output_codes(q, s, x.dtype)

@@ -1,0 +1,100 @@
+"""The direct-to-LDS dequantising GEMMs (fake-rule linears and experts) at the edges of their tiles and of
+the dispatch, against float64 on the fake-quantized tensors."""
+import pytest
+import torch
+
+from mindpipe_amd import ops
+
+pytestmark = pytest.mark.gpu
+
+DTYPES = [torch.float16, torch.bfloat16]
+# one rounding to the output dtype (half an ulp: 2^-11 / 2^-9 of a value at most, so of the norm too) and fp32
+# sums of exact products (K 2^-24 of the sum of magnitudes, a few 1e-5 of the result at these K)
+TOL = {torch.float16: 2.0 ** -11 + 5e-5, torch.bfloat16: 2.0 ** -9 + 5e-5}
+
+
+def _fake(t):
+    s = t.abs().amax(-1, keepdim=True).clamp(min=1e-5) / 127
+    return (t / s).round() * s
+
+
+def _weight(shape, dtype, gen):
+    q = torch.randint(-127, 128, shape, generator=gen, device="cuda", dtype=torch.int8)
+    s = (torch.rand(shape[:-1], generator=gen, device="cuda") * 1e-3 + 5e-4).to(dtype).float()
+    return q, s, (q.float() * s.unsqueeze(-1)).to(dtype).double()
+
+
+def _rel(a, b):
+    return float((a.double() - b).norm() / b.norm())
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("m,n,k", [
+    (1, 40, 512), (16, 4097, 640), (17, 8200, 896), (32, 16500, 512),           # a few rows: column tiles, tails, K ranges
+    (32, 264, 448), (33, 264, 512), (64, 136, 64), (65, 130, 576),              # the tiled kernel: odd steps, ragged N
+    (160, 520, 1024), (161, 392, 320), (192, 136, 256), (224, 264, 128),        # stages by row tiles
+    (256, 25000, 192), (257, 12300, 128), (1000, 50000, 64),                    # 256-row column tiles, several row slots
+])
+def test_linear_edges(dtype, m, n, k):
+    gen = torch.Generator(device="cuda").manual_seed(m * 7 + n + k)
+    q, s, w = _weight((n, k), dtype, gen)
+    x = torch.randn(m, k, generator=gen, device="cuda").to(dtype)
+    b = torch.randn(n, generator=gen, device="cuda").to(dtype)
+    ref = _fake(x).double() @ w.T
+    y = ops.w8a8_linear_fake(x, q, s, None)
+    assert y.shape == (m, n) and _rel(y, ref) <= TOL[dtype]
+    assert _rel(ops.w8a8_linear_fake(x, q, s, b), ref + b.double()) <= TOL[dtype]
+    assert _rel(ops.dq_linear(x, None, q, s, b, dtype), x.double() @ w.T + b.double()) <= TOL[dtype]
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("k", [8, 24, 2056, 16384, 16392, 40000, 100])
+def test_values_equal_codes_times_scale(dtype, k):
+    """K of every row-register count, past them, and not a multiple of 8; zero, constant and +-128 rows."""
+    gen = torch.Generator(device="cuda").manual_seed(k)
+    x = torch.randn(6, k, generator=gen, device="cuda").to(dtype)
+    x[1] = 0
+    x[2] = 0.37
+    x[3, 0], x[4, k - 1] = 9.0, -9.0
+    eye_q = torch.eye(k, device="cuda", dtype=torch.int8) if k <= 2056 else None
+    q, s = ops.quant_per_token_i8(x, True)
+    if eye_q is not None:  # a unit weight returns the activations' values
+        y = ops.w8a8_linear_fake(x, eye_q, torch.ones(k, device="cuda"), None)
+        assert torch.equal(y, (q.float() * s.float().unsqueeze(-1)).to(dtype))
+    else:
+        w = torch.randint(-127, 128, (64, k), generator=gen, device="cuda", dtype=torch.int8)
+        sw = torch.full((64,), 2.0 ** -10, device="cuda")
+        ref = (q.float() * s.float().unsqueeze(-1)).to(dtype).double() @ (w.double() * 2.0 ** -10).T
+        y = ops.w8a8_linear_fake(x, w, sw, None)
+        assert float((y.double() - ref).norm()) <= TOL[dtype] * float(ref.norm())
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("t,e,top,h,inter", [(1, 4, 1, 64, 64), (37, 8, 2, 192, 320), (300, 4, 2, 128, 576),
+                                             (700, 2, 1, 256, 192), (64, 32, 4, 512, 128)])
+def test_experts_equal_the_separate_steps(dtype, t, e, top, h, inter):
+    """The one-call chain against the four entry points on codes, with an expert no token takes and ids
+    outside [0, E): the values between the steps are the same, the sums in another order."""
+    gen = torch.Generator(device="cuda").manual_seed(t + e)
+    w13, s13, _ = _weight((e, 2 * inter, h), dtype, gen)
+    w2, s2, _ = _weight((e, h, inter), dtype, gen)
+    x = torch.randn(t, h, generator=gen, device="cuda").to(dtype)
+    ids = torch.stack([torch.randperm(e, generator=gen, device="cuda")[:top] for _ in range(t)]).to(torch.int32)
+    if e > 2:
+        ids[ids == e - 1] = -1
+    tw = torch.rand(t, top, generator=gen, device="cuda")
+    y = ops.moe_w8a8_forward(x, ids, tw, w13, s13, w2, s2, None, "fake")
+    routed, rs, slots, off = ops.moe_permute_quant(x, ids, e, "fake")
+    q, s = ops.moe_gmm1_swiglu_quant(routed, rs, w13, s13, off, inter, "fake", dtype)
+    ref = ops.moe_unpermute_combine(ops.moe_gmm2(q, s, w2, s2, off, torch.float32, "fake", dtype), slots, tw, dtype, "fake")
+    # a sum that lands on the other side of a rounding moves h by an ulp and may flip its code (1 of 127)
+    assert _rel(y, ref.double()) <= (2e-3 if dtype == torch.float16 else 8e-3)
+
+
+def test_linear_op_traces():
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    q, s, _ = _weight((72, 128), torch.bfloat16, gen)
+    x = torch.randn(2, 3, 128, generator=gen, device="cuda").bfloat16()
+    torch.library.opcheck(torch.ops.mindpipe_amd_fake.w8a8_linear.default, (x, q, s, None))
+    fn = torch.compile(lambda v: ops.w8a8_linear_fake(v, q, s, None), fullgraph=True, backend="aot_eager")
+    assert torch.equal(fn(x), ops.w8a8_linear_fake(x, q, s, None))
