@@ -113,6 +113,14 @@ int mp_w4a16_gemm(const void *x, int64_t m, int64_t k, const int32_t *w_packed, 
                   const void *scales, const void *zeros, int group_size, const void *bias, void *y,
                   int x_dtype, mp_stream_t stream);
 
+/* The same GEMM with a workspace (16-byte aligned): where M > 32 and N leave most CUs without a tile, K is split
+ * over workgroups, whose fp32 partial sums a second launch adds.  mp_w4a16_gemm_workspace_bytes: 0 where
+ * the split does not pay; with less (or no) workspace the call is mp_w4a16_gemm. */
+size_t mp_w4a16_gemm_workspace_bytes(int64_t m, int64_t n, int64_t k, int group_size);
+int mp_w4a16_gemm_ws(const void *x, int64_t m, int64_t k, const int32_t *w_packed, int64_t n,
+                     const void *scales, const void *zeros, int group_size, const void *bias,
+                     void *y, int x_dtype, void *workspace, size_t workspace_bytes, mp_stream_t stream);
+
 /* act[M, I] = silu(G) * U with [G | U] = X . dequant(W)^T (+ bias[2I]) for the fused
  * gate/up weight W [2I, K] (gate rows first): the gate/up linear and the SiLU-mul
  * of the SwiGLU MLP (act_fn(gate_up) in the HF / vLLM Llama MLP the W4A16 export
@@ -191,10 +199,10 @@ int mp_w8a8_gemm_fake(const int8_t *qx, const float *s_tok, const int8_t *w, con
                       mp_stream_t stream);
 
 /* The same linear from the activations themselves, x [M,K] in dtype (fp16 / bf16): their per-token
- * fake-quantized values r(q * s) go to the workspace (mp_w8a8_linear_fake_workspace_bytes, 16-byte
- * aligned), then y = F.linear(values, r(w * s_ch), bias) in dtype.  Equal to mp_quant_per_token_i8
+ * fake-quantized values r(q * s), and at sizes that leave CUs idle the fp32 sums of K splits, go to
+ * the workspace (mp_w8a8_linear_fake_workspace_bytes, 16-byte aligned), and y = F.linear(values, r(w * s_ch), bias) in dtype.  Equal to mp_quant_per_token_i8
  * (MP_SCALE_FAKE) followed by mp_w8a8_gemm_fake up to the order of the fp32 sums. */
-size_t mp_w8a8_linear_fake_workspace_bytes(int64_t m, int64_t k);
+size_t mp_w8a8_linear_fake_workspace_bytes(int64_t m, int64_t n, int64_t k);
 int mp_w8a8_linear_fake(const void *x, int dtype, int64_t m, int64_t k, const int8_t *w, const float *s_ch,
                         int64_t n, const void *bias, void *y, void *workspace, size_t workspace_bytes,
                         mp_stream_t stream);

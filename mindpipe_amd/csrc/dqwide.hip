@@ -13,43 +13,9 @@
 // alone, on registers, take 88 us, with operands from LDS 110, with the dequantisation 120); the Mixtral-shaped
 // experts (8 x 4096 x 14336, 512 tokens, top-2) 880 -> 566 us; M = 8, N = 11008, K = 4096 64 -> 12.6 us.
 #include "dq_wide.h"
+#include "wide_common.h"
 
 namespace {
-
-typedef __bf16 wbf8_t __attribute__((ext_vector_type(8)));
-typedef __bf16 wbf2_t __attribute__((ext_vector_type(2)));
-typedef _Float16 whf2_t __attribute__((ext_vector_type(2)));
-
-constexpr int kWBK = 64;                 // K step
-constexpr int kWLds = 160 * 1024;         // one workgroup per CU
-constexpr int kWLgkm0 = 0xC07F;          // s_waitcnt lgkmcnt(0)
-constexpr uint32_t kWOob = 0x80000000u;  // past every descriptor: zeros, no memory access
-
-// In a non-template function: with an operand that depends on a template parameter the cast to an LDS
-// pointer makes the host pass drop the kernel's launch stub.
-__device__ __forceinline__ void wide_lds_load16(__amdgpu_buffer_rsrc_t r, int8_t *lds, uint32_t voff, uint32_t soff) {
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(
-      r, reinterpret_cast<__attribute__((address_space(3))) void *>(reinterpret_cast<uintptr_t>(lds)), 16, voff,
-      __builtin_amdgcn_readfirstlane(static_cast<int>(soff)), 0, 0);
-}
-
-// The end of a phase of the K loop: nothing moves across it, in either direction.
-__device__ __forceinline__ void wide_phase() {
-  __builtin_amdgcn_sched_barrier(0);
-  asm volatile("s_barrier" ::: "memory");
-  __builtin_amdgcn_sched_barrier(0);
-}
-
-template <int DT>
-__device__ __forceinline__ uint32_t wide_pack2(float a, float b) {
-  if constexpr (DT == MP_F16) {
-    const whf2_t v = {static_cast<_Float16>(a), static_cast<_Float16>(b)};
-    return __builtin_bit_cast(uint32_t, v);
-  } else {
-    const wbf2_t v = {static_cast<__bf16>(a), static_cast<__bf16>(b)};
-    return __builtin_bit_cast(uint32_t, v);
-  }
-}
 
 // 8 int8 codes times the row scale, rounded to the dtype (q * s: one fp32 product, one conversion).
 template <int DT>
@@ -66,16 +32,6 @@ __device__ __forceinline__ uint4 wide_dq8(uint32_t w0, uint32_t w1, float s) {
     o[2 * i + 1] = wide_pack2<DT>(f2, f3);
   }
   return make_uint4(o[0], o[1], o[2], o[3]);
-}
-
-template <int DT>
-__device__ __forceinline__ f16_t wide_mfma(i4_t a, uint4 b, f16_t c) {
-  if constexpr (DT == MP_F16)
-    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(h8_t, a), __builtin_bit_cast(h8_t, b), c, 0, 0,
-                                                  0);
-  else
-    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(wbf8_t, a), __builtin_bit_cast(wbf8_t, b), c, 0,
-                                                   0, 0);
 }
 
 // Rows [rb, re) and expert of row slot `slot` (dense: the slot-th BM rows; grouped: the slot-th BM-row chunk of
@@ -122,13 +78,8 @@ __device__ __forceinline__ bool wide_rows(const mp_dq_args &p, int64_t slot, int
 // load the weights and waves 4..7 the activations: loads complete in order, so a wave that waits for
 // activations from L2 would wait for the weights it asked HBM for before them.  A phase is K = 64 where the
 // registers hold its operands, else K = 32.
-template <int N>
-__device__ __forceinline__ void wide_wait_vm() {
-  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-}
-
 template <int DT, int EPI, int TN>
-__global__ __launch_bounds__(512, 2) void dq_wide_kernel(mp_dq_args p, int n_slots) {
+__global__ __launch_bounds__(512, 2) void dq_wide_kernel(mp_dq_args p, int n_slots, int splits, float *part) {
   constexpr bool SWI = EPI == MP_EPI_SWIGLU;
   constexpr int TM = 4, WM = 2, WN = 4, BM = 256, BN = 128 * TN;
   constexpr int QB = BN / 8 / 4;  // load instructions per weight stage of a loading wave
@@ -136,7 +87,11 @@ __global__ __launch_bounds__(512, 2) void dq_wide_kernel(mp_dq_args p, int n_slo
   constexpr int CW = SWI ? 32 : 32 * TN;  // output columns of a wave
   static_assert(!SWI || TN == 2, "gate and up tiles meet in one wave");
   extern __shared__ __attribute__((aligned(16))) int8_t smem_wide[];
-  const int bx = static_cast<int>(blockIdx.x);
+  int bx = static_cast<int>(blockIdx.x), sp = 0;
+  if (TN == 1 && part) {  // the splits of a column tile sit eight apart: on one XCD
+    sp = (bx >> 3) % splits;
+    bx = (bx / (8 * splits)) * 8 + (bx & 7);
+  }
   // the row slots of a column tile sit eight apart: one XCD, whose L2 then serves their shared weights
   const int64_t col0 = (static_cast<int64_t>(bx / (8 * n_slots)) * 8 + (bx & 7)) * (SWI ? BN / 2 : BN);
   int64_t rb, re;
@@ -179,7 +134,9 @@ __global__ __launch_bounds__(512, 2) void dq_wide_kernel(mp_dq_args p, int n_slo
     const int c = colj[j] < n_out ? colj[j] : n_out - 1;
     bs[j] = p.b_scale[expert * nb_rows + c + (SWI ? j * p.n : 0)];
   }
-  const int nkt = static_cast<int>(k / kWBK), nkb = (nkt + 1) / 2;
+  // K steps [first, first + nkt) and their weight stages (a split starts and ends at a weight stage)
+  const int all = static_cast<int>(k / kWBK), first = TN == 1 ? all / 2 * sp / splits * 2 : 0;
+  const int nkt = (TN == 1 && sp + 1 < splits ? all / 2 * (sp + 1) / splits * 2 : all) - first, nkb = (nkt + 1) / 2;
   // XCDs and experts start at different places of K and wrap around: in step, every workgroup would ask for the
   // same 128 bytes of rows that lie K bytes apart, which at K = 4096 is a few of the memory channels at a time
   // (32 rows, 65536 x 4096, a start of its own for each column tile: 74 -> 59 us).  The workgroups of an XCD
@@ -191,11 +148,11 @@ __global__ __launch_bounds__(512, 2) void dq_wide_kernel(mp_dq_args p, int n_slo
   auto load_a = [&](int kt, int slot, int q) {
     const int g = q * 4 + wn;  // 8-row group
     wide_lds_load16(arsrc, smem_wide + (g < nt * 4 ? slot * ast + g * 1024 : kWLds - 1024), voff[q],
-                    wrap(kt + 2 * rot, nkt) * (kWBK * 2));
+                    (first + wrap(kt + 2 * rot, nkt)) * (kWBK * 2));
   };
   auto load_b = [&](int kb, int slot, int q) {
     wide_lds_load16(brsrc, smem_wide + b0 + slot * BST + (q * 4 + wn) * 1024, voff[q],
-                    wrap(kb + rot, nkb) * (kWBK * 2));
+                    (first + 2 * wrap(kb + rot, nkb)) * kWBK);
   };
   // at most n weight stages still in flight
   auto wait_b = [&](int n) {
@@ -337,6 +294,19 @@ __global__ __launch_bounds__(512, 2) void dq_wide_kernel(mp_dq_args p, int n_slo
   else by_rows(std::integral_constant<int, 1>{});
   asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");  // no LDS load in flight, every stage read
 
+  if constexpr (TN == 1) {
+    if (part) {
+      const int cj = c0 + wn * 32;
+#pragma unroll
+      for (int i = 0; i < TM; ++i) {
+        if (i >= nv) continue;  // wave-uniform
+        const int lr = (i * 2 + wm) * 32;
+        wide_store_part(acc[i][0], smem_wide + wave * (32 * 144), part + (sp * p.rows + rb + lr) * p.n + cj, p.n, rows - lr,
+                        n_out - cj, lane);
+      }
+      return;
+    }
+  }
   // ---- epilogue: accumulator r of tile (i, j) is row 8 (r >> 2) + 4 half + (r & 3), column lane % 32
   float bv[TN];
 #pragma unroll
@@ -380,16 +350,16 @@ __global__ __launch_bounds__(512, 2) void dq_wide_kernel(mp_dq_args p, int n_slo
 }
 
 template <int DT, int EPI, int TN>
-int wide_launch(const mp_dq_args &p, hipStream_t stream) {
+int wide_launch(const mp_dq_args &p, int splits, float *part, hipStream_t stream) {
   const int64_t slots = mp_cdiv(p.rows, 256) + (p.offsets ? p.n_experts : 0);
   const int64_t cols = mp_cdiv(mp_cdiv(p.n, EPI == MP_EPI_SWIGLU ? 64 * TN : 128 * TN), 8) * 8;
-  if (slots * cols > INT32_MAX) return MP_ERR_SHAPE;
+  if (slots * cols * splits > INT32_MAX) return MP_ERR_SHAPE;
   const void *fn = reinterpret_cast<const void *>(dq_wide_kernel<DT, EPI, TN>);
   if (hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, kWLds) != hipSuccess) return MP_ERR_HIP;
-  hipLaunchKernelGGL((dq_wide_kernel<DT, EPI, TN>), dim3(static_cast<unsigned>(slots * cols)), dim3(512), kWLds, stream, p,
-                     static_cast<int>(slots));
+  hipLaunchKernelGGL((dq_wide_kernel<DT, EPI, TN>), dim3(static_cast<unsigned>(slots * cols * splits)), dim3(512), kWLds,
+                     stream, p, static_cast<int>(slots), splits, part);
   MP_CHECK_LAUNCH();
-  return MP_OK;
+  return part ? wide_reduce<DT>(part, splits, p.rows, p.n, p.bias, p.y, stream) : MP_OK;
 }
 
 // 256 weight rows per workgroup where that makes a tile for three quarters of the CUs (half the activation reads
@@ -399,13 +369,13 @@ int wide_launch(const mp_dq_args &p, hipStream_t stream) {
 template <int DT, int EPI>
 int wide_pick(const mp_dq_args &p, hipStream_t stream) {
   if constexpr (EPI == MP_EPI_SWIGLU) {
-    return wide_launch<DT, EPI, 2>(p, stream);
+    return wide_launch<DT, EPI, 2>(p, 1, nullptr, stream);
   } else {
     const int64_t cus = mp_cu_count() > 0 ? mp_cu_count() : 256;
     const int64_t groups = p.offsets ? (p.rows < p.n_experts ? p.rows : p.n_experts) : 1;
     const int64_t tiles = mp_cdiv(p.n, 256) * groups * mp_cdiv(mp_cdiv(p.rows, groups), 256);
-    if (4 * tiles >= 3 * cus) return wide_launch<DT, EPI, 2>(p, stream);
-    return wide_launch<DT, EPI, 1>(p, stream);
+    if (4 * tiles >= 3 * cus) return wide_launch<DT, EPI, 2>(p, 1, nullptr, stream);
+    return wide_launch<DT, EPI, 1>(p, 1, nullptr, stream);
   }
 }
 
@@ -686,8 +656,16 @@ int mp_launch_dq_wide(const mp_dq_args &p, int epi, hipStream_t stream) {
 
 // SmoothQuantLinear's fake path in one call: the per-token fake-quantized activations into the workspace, then
 // the linear on them and on r(q * s) of the weight rows.
-extern "C" size_t mp_w8a8_linear_fake_workspace_bytes(int64_t m, int64_t k) {
-  return m <= 0 || k <= 0 ? 0 : static_cast<size_t>(m) * static_cast<size_t>(k) * 2;
+static int64_t mp_linear_fake_values(int64_t m, int64_t k) { return mp_cdiv(m * k * 2, 256) * 256; }
+// K splits of the linear: where the tiles leave CUs idle and the rows are past the few-row kernel's.
+static int mp_linear_fake_splits(int64_t m, int64_t n, int64_t k) {
+  return m > 32 && m < 1024 && k % 128 == 0 ? wide_splits(m, n, k) : 1;
+}
+
+extern "C" size_t mp_w8a8_linear_fake_workspace_bytes(int64_t m, int64_t n, int64_t k) {
+  if (m <= 0 || n <= 0 || k <= 0) return 0;
+  const int s = mp_linear_fake_splits(m, n, k);
+  return static_cast<size_t>(mp_linear_fake_values(m, k)) + (s > 1 ? static_cast<size_t>(s) * m * n * 4 : 0);
 }
 
 extern "C" int mp_w8a8_linear_fake(const void *x, int dtype, int64_t m, int64_t k, const int8_t *w, const float *s_ch,
@@ -697,11 +675,33 @@ extern "C" int mp_w8a8_linear_fake(const void *x, int dtype, int64_t m, int64_t 
   if (dtype != MP_F16 && dtype != MP_BF16) return MP_ERR_DTYPE;
   if (m < 0 || n <= 0 || k <= 0) return MP_ERR_SHAPE;
   if (m == 0) return MP_OK;
-  if (!workspace || workspace_bytes < mp_w8a8_linear_fake_workspace_bytes(m, k)) return MP_ERR_WORKSPACE;
+  if (!workspace || workspace_bytes < mp_w8a8_linear_fake_workspace_bytes(m, n, k)) return MP_ERR_WORKSPACE;
   if (!mp_aligned(workspace, 16)) return MP_ERR_ALIGN;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   const int rc = mp_launch_fake_values(x, dtype, m, k, nullptr, 1, workspace, s);
   if (rc != MP_OK) return rc;
+  const int splits = mp_linear_fake_splits(m, n, k);
+  if (splits > 1) {
+    mp_dq_args d{};
+    d.dt = dtype;
+    d.a = workspace;
+    d.a_fmt = MP_DQ_DT;
+    d.b = w;
+    d.b_fmt = MP_DQ_I8ROW;
+    d.b_scale = s_ch;
+    d.bias = bias;
+    d.bias_dtype = dtype;
+    d.y = y;
+    d.out_dtype = dtype;
+    d.ldy = n;
+    d.rows = m;
+    d.n = n;
+    d.k = k;
+    float *part = reinterpret_cast<float *>(static_cast<char *>(workspace) + mp_linear_fake_values(m, k));
+    if (mp_dq_wide_takes(d, MP_EPI_DENSE))
+      return dtype == MP_F16 ? wide_launch<MP_F16, MP_EPI_DENSE, 1>(d, splits, part, s)
+                             : wide_launch<MP_BF16, MP_EPI_DENSE, 1>(d, splits, part, s);
+  }
   // row parts the descriptors of every kernel of mp_dq_linear reach
   const int64_t part = mp_cdiv(int64_t(1) << 30, k) > 1 ? mp_cdiv(int64_t(1) << 30, k) - 1 : 1;
   for (int64_t r = 0; r < m; r += part) {

@@ -6,6 +6,7 @@
 // scales [N, K/g] and fp16 zeros [N, K/g] (AWQ) or an implicit zero point 8
 // (GPTQ symmetric export, stored nibble = int + 8).
 #include "dq_gemm.h"
+#include "w4_wide.h"
 
 namespace {
 
@@ -1815,6 +1816,11 @@ static bool mp_batch_takes(int64_t m, int64_t n) {
   return wgs <= 128;
 }
 
+// Whether the direct-to-LDS kernel (w4wide.hip) runs a group-128 GEMM without a workspace.
+static bool mp_w4_wide(const mp_w4_wide_args &a, bool swiglu) {
+  return mp_w4_wide_rule(a.m, a.n, swiglu) && mp_w4_wide_takes(a, swiglu);
+}
+
 // Prefill GEMM workgroup: 256 x 128 tiles of 8 waves from M = 256 (measured 8-13% faster than
 // 128 x 128 tiles of 4 waves on the 7B linears at M = 2048); MP_W4_PREFILL_THREADS=256 selects the
 // smaller tile (for measurements).
@@ -2059,6 +2065,9 @@ extern "C" int mp_w4a16_gemm_swiglu(const void *x, int64_t m, int64_t k, const i
   auto *yp = static_cast<uint16_t *>(act);
   const int ki = static_cast<int>(k), ni = static_cast<int>(n2);
   const int64_t half = n2 / 2;
+  const mp_w4_wide_args wide_args{xp, wp, sp, zp, bp, yp, x_dtype, m, n2, k};
+  if ((x_dtype == MP_BF16 || !mp_batch_takes(m, n2)) && mp_w4_wide(wide_args, true))
+    return mp_launch_w4_wide(wide_args, true, true, 1, nullptr, s);
   if (m > 64 && !mp_batch_takes(m, n2)) {
     // the prefill kernel's SwiGLU form where w4a16_gemm takes the prefill kernel (else the batched
     // kernel's SwiGLU form in row parts, below): 64 output columns (their gate and up rows) per
@@ -2204,6 +2213,12 @@ extern "C" int mp_w4a16_gemm(const void *x, int64_t m, int64_t k, const int32_t 
   if (!x || !w_packed || !scales || !y) return MP_ERR_ARG;
   if (m > INT32_MAX || n > INT32_MAX || k > INT32_MAX) return MP_ERR_SHAPE;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  if (group_size == 128) {
+    const mp_w4_wide_args a{static_cast<const uint16_t *>(x), reinterpret_cast<const uint32_t *>(w_packed),
+                            static_cast<const uint16_t *>(scales), static_cast<const uint16_t *>(zeros),
+                            static_cast<const uint16_t *>(bias), static_cast<uint16_t *>(y), x_dtype, m, n, k};
+    if (mp_w4_wide(a, false)) return mp_launch_w4_wide(a, false, !mp_batch_takes(m, n), 1, nullptr, s);
+  }
   if (x_dtype == MP_BF16) {
     // bf16: every dequantised weight rounded to bf16 as the reference's pseudo-quantized
     // weight is (bf16 keeps 8 significant bits: factoring the group scale out of the sum, as
@@ -2475,3 +2490,6 @@ extern "C" int mp_w4a16_gemm(const void *x, int64_t m, int64_t k, const int32_t 
   MP_CHECK_LAUNCH();
   return MP_OK;
 }
+
+// fp16 rows that the batched kernel takes keep its numerics (no weight is rounded), see mp_launch_w4_wide.
+bool mp_w4_batch_numerics(int64_t m, int64_t n) { return mp_batch_takes(m, n); }

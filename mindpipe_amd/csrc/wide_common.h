@@ -1,0 +1,140 @@
+// Device helpers of the direct-to-LDS GEMMs (dqwide.hip, w4wide.hip).
+#pragma once
+#include "mp_common.h"
+
+namespace {
+
+typedef __bf16 wbf8_t __attribute__((ext_vector_type(8)));
+typedef __bf16 wbf2_t __attribute__((ext_vector_type(2)));
+typedef _Float16 whf2_t __attribute__((ext_vector_type(2)));
+
+constexpr int kWBK = 64;                 // K step
+constexpr int kWLds = 160 * 1024;         // one workgroup per CU
+constexpr int kWLgkm0 = 0xC07F;          // s_waitcnt lgkmcnt(0)
+constexpr uint32_t kWOob = 0x80000000u;  // past every descriptor: zeros, no memory access
+
+// In a non-template function: with an operand that depends on a template parameter the cast to an LDS
+// pointer makes the host pass drop the kernel's launch stub.
+__device__ __forceinline__ void wide_lds_load16(__amdgpu_buffer_rsrc_t r, int8_t *lds, uint32_t voff, uint32_t soff) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(
+      r, reinterpret_cast<__attribute__((address_space(3))) void *>(reinterpret_cast<uintptr_t>(lds)), 16, voff,
+      __builtin_amdgcn_readfirstlane(static_cast<int>(soff)), 0, 0);
+}
+
+// The end of a phase of the K loop: nothing moves across it, in either direction.
+__device__ __forceinline__ void wide_phase() {
+  __builtin_amdgcn_sched_barrier(0);
+  asm volatile("s_barrier" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+}
+
+template <int DT>
+__device__ __forceinline__ uint32_t wide_pack2(float a, float b) {
+  if constexpr (DT == MP_F16) {
+    const whf2_t v = {static_cast<_Float16>(a), static_cast<_Float16>(b)};
+    return __builtin_bit_cast(uint32_t, v);
+  } else {
+    const wbf2_t v = {static_cast<__bf16>(a), static_cast<__bf16>(b)};
+    return __builtin_bit_cast(uint32_t, v);
+  }
+}
+
+template <int DT>
+__device__ __forceinline__ f16_t wide_mfma(i4_t a, uint4 b, f16_t c) {
+  if constexpr (DT == MP_F16)
+    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(h8_t, a), __builtin_bit_cast(h8_t, b), c, 0, 0,
+                                                  0);
+  else
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(wbf8_t, a), __builtin_bit_cast(wbf8_t, b), c, 0,
+                                                   0, 0);
+}
+
+template <int N>
+__device__ __forceinline__ void wide_wait_vm() {
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+
+// One 32 x 32 fp32 MFMA tile of a K split to the partials, through a wave-private LDS tile of 144-byte rows:
+// accumulator r is row 8 (r >> 2) + 4 half + (r & 3), column lane % 32; a lane then stores four columns of a row.
+// `rows` and `cols` bound what is stored of the tile, `ld` is the row stride (elements), dst the tile's corner.
+__device__ __forceinline__ void wide_store_part(const f16_t &acc, int8_t *stage, float *dst, int64_t ld, int rows, int cols,
+                                                int lane) {
+#pragma unroll
+  for (int r = 0; r < 16; ++r)
+    *reinterpret_cast<float *>(stage + (8 * (r >> 2) + 4 * (lane >> 5) + (r & 3)) * 144 + (lane & 31) * 4) = acc[r];
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const int row = q * 8 + lane / 8, col = (lane & 7) * 4;
+    const f4_t v = *reinterpret_cast<const f4_t *>(stage + row * 144 + (lane & 7) * 16);
+    if (row >= rows) continue;
+    float *d = dst + row * ld + col;
+    if (ld % 4 == 0) {
+      if (col < cols) *reinterpret_cast<f4_t *>(d) = v;
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (col + e < cols) d[e] = v[e];
+    }
+  }
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the next tile overwrites the region
+}
+
+// Sums of the K splits' fp32 partials [splits, m, n] in split order, plus bias, rounded once; four columns per thread.
+template <int DT>
+__global__ __launch_bounds__(256) void wide_reduce_kernel(const float *__restrict__ part, int splits, int64_t m, int64_t n,
+                                                          const uint16_t *__restrict__ bias, uint16_t *__restrict__ y) {
+  const int64_t per = (n + 3) / 4, t = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+  if (t >= m * per) return;
+  const int64_t row = t / per, c = t % per * 4;
+  float v[4] = {0.f, 0.f, 0.f, 0.f};
+  for (int s = 0; s < splits; ++s) {
+    const float *src = part + (s * m + row) * n + c;
+    if (n % 4 == 0) {
+      const float4 w = *reinterpret_cast<const float4 *>(src);
+      v[0] = mp_add(v[0], w.x);
+      v[1] = mp_add(v[1], w.y);
+      v[2] = mp_add(v[2], w.z);
+      v[3] = mp_add(v[3], w.w);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (c + e < n) v[e] = mp_add(v[e], src[e]);
+    }
+  }
+  uint16_t o[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const float f = bias && c + e < n ? mp_add(v[e], mp_load_as_f32(bias, c + e, DT)) : v[e];
+    o[e] = DT == MP_F16 ? mp_f2h(f) : mp_f2bf(f);
+  }
+  uint16_t *d = y + row * n + c;
+  if (n % 4 == 0 && (reinterpret_cast<uintptr_t>(y) & 7) == 0) {
+    *reinterpret_cast<uint2 *>(d) = make_uint2(o[0] | (static_cast<uint32_t>(o[1]) << 16), o[2] | (static_cast<uint32_t>(o[3]) << 16));
+  } else {
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (c + e < n) d[e] = o[e];
+  }
+}
+
+// Ways to split K over workgroups so that tiles of 256 rows x 128 columns give each CU one: at least K = 1024
+// each, at most 8.
+inline int wide_splits(int64_t m, int64_t n, int64_t k) {
+  const int64_t cus = mp_cu_count() > 0 ? mp_cu_count() : 256;
+  const int64_t tiles = mp_cdiv(n, 128) * mp_cdiv(m, 256);
+  int64_t s = cus / tiles;
+  if (s > k / 1024) s = k / 1024;
+  if (s > 8) s = 8;
+  return s < 1 ? 1 : static_cast<int>(s);
+}
+
+template <int DT>
+int wide_reduce(const float *part, int splits, int64_t m, int64_t n, const void *bias, void *y, hipStream_t stream) {
+  hipLaunchKernelGGL((wide_reduce_kernel<DT>), dim3(static_cast<unsigned>(mp_cdiv(m * mp_cdiv(n, 4), 256))), dim3(256), 0,
+                     stream, part, splits, m, n, static_cast<const uint16_t *>(bias), static_cast<uint16_t *>(y));
+  MP_CHECK_LAUNCH();
+  return MP_OK;
+}
+
+}  // namespace

@@ -150,10 +150,13 @@ def w4a16_gemm(x: torch.Tensor, w_packed: torch.Tensor, scales: torch.Tensor, ze
     x2 = x.reshape(-1, k)
     m = x2.shape[0]
     y = torch.empty((m, n), dtype=x.dtype, device=x.device)
+    lib = _lib.load()
+    wsb = lib.mp_w4a16_gemm_workspace_bytes(m, n, k, group_size) if m > 32 else 0
+    ws = torch.empty((wsb,), dtype=torch.uint8, device=x.device) if wsb else None
     with _dev(x):
-        _lib.check(_lib.load().mp_w4a16_gemm(
+        _lib.check(lib.mp_w4a16_gemm_ws(
             x2.data_ptr(), m, k, w_packed.data_ptr(), n, scales.data_ptr(), _ptr(zeros), group_size,
-            _ptr(bias), y.data_ptr(), _DT[x.dtype], _stream()), "mp_w4a16_gemm")
+            _ptr(bias), y.data_ptr(), _DT[x.dtype], _ptr(ws), wsb, _stream()), "mp_w4a16_gemm_ws")
     return y.reshape(*x.shape[:-1], n)
 
 
@@ -392,11 +395,13 @@ def w8a8_linear_fake(x: torch.Tensor, w: torch.Tensor, s_ch: torch.Tensor,
     x2 = x.reshape(-1, k)
     m = x2.shape[0]
     y = torch.empty((*x.shape[:-1], n), dtype=x.dtype, device=x.device)
-    ws = torch.empty((m, k), dtype=x.dtype, device=x.device)
+    lib = _lib.load()
+    wsb = lib.mp_w8a8_linear_fake_workspace_bytes(m, n, k)
+    ws = torch.empty((wsb,), dtype=torch.uint8, device=x.device)
     with _dev(x):
-        _lib.check(_lib.load().mp_w8a8_linear_fake(
+        _lib.check(lib.mp_w8a8_linear_fake(
             x2.data_ptr(), _DT[x.dtype], m, k, w.data_ptr(), s_ch.data_ptr(), n, _ptr(bias), y.data_ptr(),
-            ws.data_ptr(), ws.numel() * 2, _stream()), "mp_w8a8_linear_fake")
+            ws.data_ptr(), wsb, _stream()), "mp_w8a8_linear_fake")
     return y
 
 

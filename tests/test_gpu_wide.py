@@ -1,0 +1,63 @@
+"""The direct-to-LDS W4A16 and int8 GEMMs at the edges of their tiles, of the K split and of the dispatch: the int8 ones
+bit for bit against the exact product with the epilogue's operations, the W4A16 ones against float64."""
+import pytest
+import torch
+
+from mindpipe_amd import ops
+
+pytestmark = pytest.mark.gpu
+
+DTYPES = [torch.float16, torch.bfloat16]
+# one rounding of the output (half an ulp of a value at most) and of every weight where the kernel rounds them (the sum of
+# K such errors is at most that share of the result's norm), and fp32 sums
+TOL = {torch.float16: 2 * 2.0 ** -11 + 5e-5, torch.bfloat16: 2 * 2.0 ** -9 + 5e-5}
+
+
+def _gen(*key):
+    return torch.Generator(device="cuda").manual_seed(sum(k * p for k, p in zip(key, (1, 1009, 9176, 31))))
+
+
+def _w4(n, k, dtype, gen, zeros=True):
+    packed = torch.randint(-2 ** 31, 2 ** 31 - 1, (n, k // 8), generator=gen, device="cuda", dtype=torch.int64).to(torch.int32)
+    s = (torch.rand(n, k // 128, generator=gen, device="cuda") * 0.004 + 0.004).to(dtype)
+    z = torch.randint(0, 16, (n, k // 128), generator=gen, device="cuda").to(dtype) if zeros else None
+    u = ((packed.unsqueeze(-1) >> torch.arange(0, 32, 4, device="cuda", dtype=torch.int32)) & 15).flatten(1).double()
+    zz = z.double() if zeros else torch.full_like(s, 8).double()
+    w = (u - zz.repeat_interleave(128, 1)) * s.double().repeat_interleave(128, 1)
+    return packed, s, z, w
+
+
+def _rel(a, b):
+    return float((a.double() - b).norm() / b.norm())
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("m,n,k,zeros", [
+    (65, 12290, 256, True), (96, 12288, 512, False), (130, 12300, 768, True),   # no workspace: 96 tiles and up, ragged N
+    (257, 6200, 256, True), (600, 8192, 512, True), (1025, 2568, 1024, False),   # several row slots, one of one row
+    (77, 13824, 5120, True), (33, 16392, 8192, False), (200, 4100, 8192, True),  # K split: 2, 1 and 7 ways
+    (256, 4096, 4096, True), (1023, 1032, 4352, True), (64, 8200, 9216, True),
+    (64, 4096, 512, True), (80, 520, 640, True),                                 # the kernels below the rules
+])
+def test_w4_linear(dtype, m, n, k, zeros):
+    gen = _gen(m, n, k)
+    packed, s, z, w = _w4(n, k, dtype, gen, zeros)
+    x = torch.randn(m, k, generator=gen, device="cuda").to(dtype)
+    b = torch.randn(n, generator=gen, device="cuda").to(dtype)
+    ref = x.double() @ w.T
+    assert _rel(ops.w4a16_gemm(x, packed, s, z, 128, None), ref) <= TOL[dtype]
+    assert _rel(ops.w4a16_gemm(x, packed, s, z, 128, b), ref + b.double()) <= TOL[dtype]
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("m,n2,k", [(65, 12544, 256), (200, 12304, 512), (300, 6208, 768), (513, 8200, 256), (66, 256, 512)])
+def test_w4_swiglu(dtype, m, n2, k):
+    """Gate and up in one kernel against the two launches: the same roundings, sums in another order (an output moves by
+    a few ulps where gate, up or silu lands on the other side of one)."""
+    gen = _gen(m, n2, k)
+    packed, s, z, _ = _w4(n2, k, dtype, gen)
+    x = torch.randn(m, k, generator=gen, device="cuda").to(dtype)
+    b = torch.randn(n2, generator=gen, device="cuda").to(dtype)
+    y = ops.w4a16_gemm_swiglu(x, packed, s, z, 128, b)
+    ref = ops.silu_mul(ops.w4a16_gemm(x, packed, s, z, 128, b))
+    assert y.shape == (m, n2 // 2) and _rel(y, ref.double()) <= 2 * TOL[dtype]
