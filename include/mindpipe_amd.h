@@ -187,6 +187,15 @@ int mp_w8a8_gemm(const int8_t *qx, const float *s_tok, const int8_t *w, const fl
                  const void *bias, int bias_dtype, void *y, int out_dtype, int64_t m, int64_t n,
                  int64_t k, mp_stream_t stream);
 
+/* The same GEMM with a workspace (16-byte aligned): at row counts and widths that leave most CUs
+ * without a tile, K is split over workgroups and the exact int32 partial sums are added by a second
+ * launch.  The outputs are the same bits.  mp_w8a8_gemm_workspace_bytes: 0 where the split does not
+ * pay; with less (or no) workspace the call is mp_w8a8_gemm. */
+size_t mp_w8a8_gemm_workspace_bytes(int64_t m, int64_t n, int64_t k);
+int mp_w8a8_gemm_ws(const int8_t *qx, const float *s_tok, const int8_t *w, const float *s_ch,
+                    const void *bias, int bias_dtype, void *y, int out_dtype, int64_t m, int64_t n,
+                    int64_t k, void *workspace, size_t workspace_bytes, mp_stream_t stream);
+
 /* y[M,N] = F.linear(r(qx * s_tok), r(w * s_ch), bias) in act_dtype (fp16 / bf16): the
  * fake path of SmoothQuantLinear.forward (fake_quant.py:85-88) on the fake rule's codes
  * (MP_SCALE_FAKE of mp_quant_per_token_i8 / mp_w8_quantize_per_channel), each operand

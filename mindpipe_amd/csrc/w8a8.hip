@@ -1,6 +1,7 @@
 // W8A8 for gfx950: per-token / per-channel int8 quantizers and the int8 MFMA
 // GEMM with the per-token x per-channel scale epilogue (dense and grouped).
 #include "dq_gemm.h"
+#include "i8_wide.h"
 #include <type_traits>
 
 namespace {
@@ -2179,7 +2180,30 @@ static int mp_launch_moe(const mp_i8_args &a, hipStream_t stream) {
 }
 
 // Shared launcher (dense + grouped).
+// Whether the direct-to-LDS kernel (i8wide.hip) is the faster one.  Graph-timed calls with the row quant:
+//   dense, M >= 1024, against the large-M kernel: M = 2048, 4096 x 4096 56 against 77 us, M = 2000, N = 4096, K = 11008 128
+//   against 192 us, M = 1500, 8192 x 8192 130 against 156 us, M = 4096, N = 11008 234 against 237 us;
+//   dense, 33 <= M < 1024, from 96 tiles of 256 rows x 128 columns (80 up to 64 rows) where the mid-M kernel does not
+//   run: M = 800, 8192 x 8192 86 against 109 us, M = 512, N = 11008 46 against 54 us, M = 64, N = 11008 / 28672 26.5 / 35
+//   against 31 / 44 us (the mid-M kernel's smaller tiles win at M = 256, N = 11008: 29 against 39 us);
+//   grouped, from three tiles for four CUs, against i8_moe_kernel: the Mixtral-shaped chain at 4 / 16 / 48 / 512 /
+//   1000 tokens 227 / 306 / 309 / 412 / 667 against 283 / 337 / 344 / 457 / 744 us (one group of 200 rows, I = 11008: 86
+//   tiles, GEMM1 63 against 46 us).
+static bool mp_wide_takes(const mp_i8_args &a, int epilogue) {
+  if (epilogue == MP_EPI_AMAX || !mp_i8_wide_takes(a, epilogue)) return false;
+  const int64_t cus = mp_cu_count() > 0 ? mp_cu_count() : 256;
+  if (a.offsets) {
+    const int64_t groups = a.rows < a.n_experts ? a.rows : a.n_experts;
+    return 4 * mp_cdiv(a.n, 128) * groups * mp_cdiv(mp_cdiv(a.rows, groups), 256) >= 3 * cus;
+  }
+  if (epilogue != MP_EPI_DENSE || a.rows <= 32) return false;
+  if (a.rows >= 1024) return true;
+  const int64_t tiles = mp_cdiv(a.n, 128) * mp_cdiv(a.rows, 256);
+  return a.rows <= 64 ? tiles >= 80 : (mp_mid_bn(a) == 0 && tiles >= 96);
+}
+
 int mp_launch_i8_gemm(const mp_i8_args &a, int epilogue, hipStream_t stream) {
+  if (mp_wide_takes(a, epilogue)) return mp_launch_i8_wide(a, epilogue, stream);
   // the tiled kernel addresses a tile's 128 output rows, and its 128 activation rows, through one
   // descriptor each
   const bool aligned = mp_aligned(a.a, 16) && mp_aligned(a.b, 16) && a.ldy < (int64_t(1) << 23) &&
@@ -2541,6 +2565,41 @@ extern "C" int mp_w8a8_gemm(const int8_t *qx, const float *s_tok, const int8_t *
   a.k = k;
   a.ldy = n;
   return mp_launch_i8_gemm(a, MP_EPI_DENSE, reinterpret_cast<hipStream_t>(stream));
+}
+
+extern "C" size_t mp_w8a8_gemm_workspace_bytes(int64_t m, int64_t n, int64_t k) {
+  // K split where K is long or the rows few: measured (graph-timed calls with the row quant) against the kernels
+  // without it M = 200, N = 4096, K = 11008 38 against 56 us, M = 100, 8192 x 8192 36 against 47 us, M = 64, N = 8192, K = 28672
+  // 74 against 163 us, M = 40, 4096 x 4096 18 against 21 us; M = 256, 4096 x 4096 26 against 23 us
+  if (m <= 32 || m >= 1024 || n <= 0 || k <= 0 || k % 128 != 0 || (k < 8192 && m > 64)) return 0;
+  const int s = mp_i8_wide_splits(m, n, k);
+  return s < 2 ? 0 : static_cast<size_t>(s) * static_cast<size_t>(m) * static_cast<size_t>(n) * sizeof(int);
+}
+
+extern "C" int mp_w8a8_gemm_ws(const int8_t *qx, const float *s_tok, const int8_t *w, const float *s_ch,
+                               const void *bias, int bias_dtype, void *y, int out_dtype, int64_t m, int64_t n,
+                               int64_t k, void *workspace, size_t workspace_bytes, mp_stream_t stream) {
+  const size_t need = mp_w8a8_gemm_workspace_bytes(m, n, k);
+  mp_i8_args a{};
+  a.a = qx;
+  a.s_a = s_tok;
+  a.b = w;
+  a.s_b = s_ch;
+  a.bias = bias;
+  a.bias_dtype = bias_dtype;
+  a.y = y;
+  a.out_dtype = out_dtype;
+  a.rows = m;
+  a.n = n;
+  a.k = k;
+  a.ldy = n;
+  if (need == 0 || !workspace || workspace_bytes < need || !mp_aligned(workspace, 16) || !qx || !s_tok || !w || !s_ch || !y ||
+      k > (1 << 17) || !mp_i8_wide_takes(a, MP_EPI_DENSE) ||
+      (out_dtype != MP_F16 && out_dtype != MP_BF16 && out_dtype != MP_F32) ||
+      (bias && bias_dtype != MP_F16 && bias_dtype != MP_BF16 && bias_dtype != MP_F32))
+    return mp_w8a8_gemm(qx, s_tok, w, s_ch, bias, bias_dtype, y, out_dtype, m, n, k, stream);
+  return mp_launch_i8_split(a, mp_i8_wide_splits(m, n, k), static_cast<int *>(workspace),
+                            reinterpret_cast<hipStream_t>(stream));
 }
 
 extern "C" int mp_w8a8_gemm_fake(const int8_t *qx, const float *s_tok, const int8_t *w, const float *s_ch,

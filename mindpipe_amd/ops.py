@@ -326,11 +326,14 @@ def w8a8_gemm(qx: torch.Tensor, s_tok: torch.Tensor, w: torch.Tensor, s_ch: torc
     if bias is not None:
         _need(bias, "bias", (torch.float16, torch.bfloat16, torch.float32), 1)
     y = torch.empty((m, n), dtype=out_dtype, device=qx.device)
+    lib = _lib.load()
+    wsb = lib.mp_w8a8_gemm_workspace_bytes(m, n, k)
+    ws = torch.empty((wsb,), dtype=torch.uint8, device=qx.device) if wsb else None
     with _dev(qx):
-        _lib.check(_lib.load().mp_w8a8_gemm(
+        _lib.check(lib.mp_w8a8_gemm_ws(
             q2.data_ptr(), s_tok.data_ptr(), w.data_ptr(), s_ch.data_ptr(), _ptr(bias),
-            _DT[bias.dtype] if bias is not None else MP_F16, y.data_ptr(), _DT[out_dtype], m, n, k, _stream()),
-            "mp_w8a8_gemm")
+            _DT[bias.dtype] if bias is not None else MP_F16, y.data_ptr(), _DT[out_dtype], m, n, k, _ptr(ws), wsb,
+            _stream()), "mp_w8a8_gemm_ws")
     return y.reshape(*qx.shape[:-1], n)
 
 

@@ -61,3 +61,51 @@ def test_w4_swiglu(dtype, m, n2, k):
     y = ops.w4a16_gemm_swiglu(x, packed, s, z, 128, b)
     ref = ops.silu_mul(ops.w4a16_gemm(x, packed, s, z, 128, b))
     assert y.shape == (m, n2 // 2) and _rel(y, ref.double()) <= 2 * TOL[dtype]
+
+
+@pytest.mark.parametrize("out", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("m,n,k", [
+    (33, 10300, 256), (64, 10240, 128), (65, 24600, 384), (513, 11010, 256),     # 80 / 96 tiles and up, ragged N
+    (1024, 130, 128), (1025, 520, 640), (1300, 4096, 1280),                       # every M from 1024
+    (200, 4100, 8192), (40, 4096, 4096), (1000, 1001, 9216), (64, 8192, 28672),   # K split
+    (256, 4096, 4096), (100, 520, 1024),                                          # the kernels below the rules
+])
+def test_int8_linear_bits(out, m, n, k):
+    gen = _gen(m, n, k)
+    q = torch.randint(-127, 128, (m, k), generator=gen, device="cuda", dtype=torch.int8)
+    w = torch.randint(-127, 128, (n, k), generator=gen, device="cuda", dtype=torch.int8)
+    st, sc = torch.rand(m, generator=gen, device="cuda") * 0.01, torch.rand(n, generator=gen, device="cuda") * 0.01
+    b = torch.randn(n, generator=gen, device="cuda").to(out)
+    acc = (q.double() @ w.double().T).float()
+    ref = ((acc * st[:, None]) * sc[None]) + b.float()
+    assert torch.equal(ops.w8a8_gemm(q, st, w, sc, b, out), ref.to(out))
+    assert torch.equal(ops.w8a8_gemm(q, st, w, sc, None, out), ((acc * st[:, None]) * sc[None]).to(out))
+
+
+@pytest.mark.parametrize("t,e,top,h,inter", [(1, 64, 1, 128, 448), (48, 8, 2, 256, 3136), (700, 8, 2, 3200, 1536),
+                                             (300, 2, 1, 12416, 12352), (64, 32, 4, 3072, 896)])
+def test_int8_experts_bits(t, e, top, h, inter):
+    """GEMM1 + SwiGLU + requant and GEMM2 over groups of 0 to 350 rows: GEMM2 bit for bit; the codes up to those that
+    exp's last bit decides."""
+    gen = _gen(t, e, h, inter)
+    w13 = torch.randint(-127, 128, (e, 2 * inter, h), generator=gen, device="cuda", dtype=torch.int8)
+    s13 = torch.rand(e, 2 * inter, generator=gen, device="cuda") * 1e-3
+    w2 = torch.randint(-127, 128, (e, h, inter), generator=gen, device="cuda", dtype=torch.int8)
+    s2 = torch.rand(e, h, generator=gen, device="cuda") * 1e-3
+    x = torch.randn(t, h, generator=gen, device="cuda").half()
+    ids = torch.stack([torch.randperm(e, generator=gen, device="cuda")[:top] for _ in range(t)]).int()
+    routed, rs, _, off = ops.moe_permute_quant(x, ids, e)
+    q, s = ops.moe_gmm1_swiglu_quant(routed, rs, w13, s13, off, inter)
+    y = ops.moe_gmm2(q, s, w2, s2, off)
+    differ = 0
+    ends = off.tolist()
+    for i in range(e):
+        a, b = ends[i], ends[i + 1]
+        if a == b:
+            continue
+        gu = ((routed[a:b].double() @ w13[i].double().T).float() * rs[a:b, None]) * s13[i][None]
+        g, u = gu[:, :inter], gu[:, inter:]
+        hh = g / (1 + torch.exp(-g)) * u
+        differ += int(((hh / (hh.abs().amax(-1, keepdim=True) / 127)).round().to(torch.int8) != q[a:b]).sum())
+        assert torch.equal(((q[a:b].double() @ w2[i].double().T).float() * s[a:b, None]) * s2[i][None], y[a:b])
+    assert differ <= 1e-3 * q.numel()
