@@ -196,6 +196,13 @@ int mp_w8a8_gemm_ws(const int8_t *qx, const float *s_tok, const int8_t *w, const
                     const void *bias, int bias_dtype, void *y, int out_dtype, int64_t m, int64_t n,
                     int64_t k, void *workspace, size_t workspace_bytes, mp_stream_t stream);
 
+/* mp_quant_per_token_i8 (scale_rule) of x [M,K] and the GEMM on its codes, in one call and with the same bits: codes,
+ * fp32 scales and the GEMM's own workspace in `workspace` (mp_w8a8_linear_workspace_bytes, 16-byte aligned). */
+size_t mp_w8a8_linear_workspace_bytes(int64_t m, int64_t n, int64_t k);
+int mp_w8a8_linear(const void *x, int x_dtype, int64_t m, int64_t k, const int8_t *w, const float *s_ch, int64_t n,
+                   const void *bias, int bias_dtype, void *y, int out_dtype, int scale_rule, void *workspace,
+                   size_t workspace_bytes, mp_stream_t stream);
+
 /* y[M,N] = F.linear(r(qx * s_tok), r(w * s_ch), bias) in act_dtype (fp16 / bf16): the
  * fake path of SmoothQuantLinear.forward (fake_quant.py:85-88) on the fake rule's codes
  * (MP_SCALE_FAKE of mp_quant_per_token_i8 / mp_w8_quantize_per_channel), each operand

@@ -64,6 +64,8 @@ SIGNATURES = {
     "mp_w4a16_gemm_ws": (_i32, [_vp, _i64, _i64, _vp, _i64, _vp, _vp, _i32, _vp, _vp, _i32, _vp, C.c_size_t, _vp]),
     "mp_w8a8_gemm_workspace_bytes": (C.c_size_t, [_i64, _i64, _i64]),
     "mp_w8a8_gemm_ws": (_i32, [_vp, _vp, _vp, _vp, _vp, _i32, _vp, _i32, _i64, _i64, _i64, _vp, C.c_size_t, _vp]),
+    "mp_w8a8_linear_workspace_bytes": (C.c_size_t, [_i64, _i64, _i64]),
+    "mp_w8a8_linear": (_i32, [_vp, _i32, _i64, _i64, _vp, _vp, _i64, _vp, _i32, _vp, _i32, _i32, _vp, C.c_size_t, _vp]),
     "mp_w8a8_linear_fake_workspace_bytes": (C.c_size_t, [_i64, _i64, _i64]),
     "mp_w8a8_linear_fake": (_i32, [_vp, _i32, _i64, _i64, _vp, _vp, _i64, _vp, _vp, _vp, C.c_size_t, _vp]),
     "mp_moe_fake_workspace_bytes": (C.c_size_t, [_i64, _i64, _i64, _i32, _i32]),

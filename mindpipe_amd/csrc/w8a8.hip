@@ -2602,6 +2602,39 @@ extern "C" int mp_w8a8_gemm_ws(const int8_t *qx, const float *s_tok, const int8_
                             reinterpret_cast<hipStream_t>(stream));
 }
 
+static size_t mp_w8a8_linear_codes(int64_t m, int64_t k) { return static_cast<size_t>(mp_cdiv(m * k, 256) * 256); }
+static size_t mp_w8a8_linear_scales(int64_t m) { return static_cast<size_t>(mp_cdiv(m * 4, 256) * 256); }
+
+extern "C" size_t mp_w8a8_linear_workspace_bytes(int64_t m, int64_t n, int64_t k) {
+  if (m <= 0 || n <= 0 || k <= 0) return 0;
+  return mp_w8a8_linear_codes(m, k) + mp_w8a8_linear_scales(m) + mp_w8a8_gemm_workspace_bytes(m, n, k);
+}
+
+extern "C" int mp_w8a8_linear(const void *x, int x_dtype, int64_t m, int64_t k, const int8_t *w, const float *s_ch,
+                              int64_t n, const void *bias, int bias_dtype, void *y, int out_dtype, int scale_rule,
+                              void *workspace, size_t workspace_bytes, mp_stream_t stream) {
+  if (!x || !w || !s_ch || !y) return MP_ERR_ARG;
+  if (x_dtype != MP_F16 && x_dtype != MP_BF16 && (x_dtype != MP_F32 || scale_rule != MP_SCALE_FP32)) return MP_ERR_DTYPE;
+  if (out_dtype != MP_F16 && out_dtype != MP_BF16 && out_dtype != MP_F32) return MP_ERR_DTYPE;
+  if (bias && bias_dtype != MP_F16 && bias_dtype != MP_BF16 && bias_dtype != MP_F32) return MP_ERR_DTYPE;
+  if (scale_rule != MP_SCALE_FP32 && scale_rule != MP_SCALE_FAKE) return MP_ERR_ARG;
+  if (m < 0 || m > INT32_MAX || n <= 0 || k <= 0 || k > (1 << 17)) return MP_ERR_SHAPE;
+  if (m == 0) return MP_OK;
+  if (!workspace || workspace_bytes < mp_w8a8_linear_workspace_bytes(m, n, k)) return MP_ERR_WORKSPACE;
+  if (!mp_aligned(workspace, 16)) return MP_ERR_ALIGN;
+  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  auto *q = static_cast<int8_t *>(workspace);
+  auto *st = reinterpret_cast<float *>(q + mp_w8a8_linear_codes(m, k));
+  if (scale_rule == MP_SCALE_FP32)
+    mp_launch_rowquant<MP_SCALE_FP32>(x, x_dtype, m, k, q, st, nullptr, 0, 0.0f, nullptr, s);
+  else
+    mp_launch_rowquant<MP_SCALE_FAKE>(x, x_dtype, m, k, q, st, nullptr, 0, 0.0f, nullptr, s);
+  MP_CHECK_LAUNCH();
+  return mp_w8a8_gemm_ws(q, st, w, s_ch, bias, bias_dtype, y, out_dtype, m, n, k,
+                         reinterpret_cast<char *>(st) + mp_w8a8_linear_scales(m), mp_w8a8_gemm_workspace_bytes(m, n, k),
+                         stream);
+}
+
 extern "C" int mp_w8a8_gemm_fake(const int8_t *qx, const float *s_tok, const int8_t *w, const float *s_ch,
                                  const void *bias, int act_dtype, void *y, int64_t m, int64_t n, int64_t k,
                                  mp_stream_t stream) {

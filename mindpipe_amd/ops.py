@@ -22,7 +22,7 @@ _DT = {torch.float16: MP_F16, torch.bfloat16: MP_BF16, torch.float32: MP_F32}
 
 
 def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
@@ -42,8 +42,63 @@ def _need(t: torch.Tensor, name: str, dtype=None, ndim=None) -> None:
         raise RuntimeError(f"{name} must be contiguous")
 
 
+class _SameDevice:
+    """The device is current already: nothing to switch (entering ``torch.cuda.device`` costs microseconds)."""
+
+    def __enter__(self):
+        return None
+
+    def __exit__(self, *exc):
+        return False
+
+
+_SAME_DEVICE = _SameDevice()
+
+
 def _dev(t: torch.Tensor):
-    return torch.cuda.device(t.device)
+    return _SAME_DEVICE if t.device.index == torch._C._cuda_getDevice() else torch.cuda.device(t.device)
+
+
+# ---------------------------------------------------------------- registration
+_LIGHT = torch.library.Library("mindpipe_amd_light", "DEF")
+
+
+class _Op:
+    """An op registered twice over one function: as the custom op ``torch.ops.mindpipe_amd.<name>`` and, without that
+    wrapper's Python autograd layer, as ``torch.ops.mindpipe_amd_light.<name>`` with the same fake implementation.
+    A call goes to the custom op under compilation, functorch transforms and forward-mode AD and where an
+    input requires a gradient (it refuses the backward); otherwise to the light one: the custom op's layers cost
+    about 11 us a call, half of an eager one-row linear (23 us)."""
+
+    def __init__(self, fn, name, ns):
+        self.fn, self.name, self.__doc__, self.__name__ = fn, name, fn.__doc__, fn.__name__
+        self.def_ = torch.library.custom_op(f"{ns}::{name}", mutates_args=())(fn)
+        _LIGHT.define(name + torch.library.infer_schema(fn, mutates_args=()))
+        _LIGHT.impl(name, fn, "CompositeExplicitAutograd")
+        self.full = getattr(getattr(torch.ops, ns), name).default
+        self.light = getattr(torch.ops.mindpipe_amd_light, name).default
+
+    def register_fake(self, fake):
+        self.def_.register_fake(fake)
+        torch.library.register_fake(f"mindpipe_amd_light::{self.name}", fake, lib=_LIGHT)
+        return fake
+
+    def __call__(self, *args, **kwargs):
+        if (torch.compiler.is_compiling() or torch._C._functorch.peek_interpreter_stack() is not None
+                or torch.autograd.forward_ad._current_level >= 0):
+            return self.full(*args, **kwargs)
+        if torch.is_grad_enabled():
+            for a in (*args, *kwargs.values()):
+                if isinstance(a, torch.Tensor):
+                    if a.requires_grad:
+                        return self.full(*args, **kwargs)
+                elif isinstance(a, (list, tuple)) and any(isinstance(t, torch.Tensor) and t.requires_grad for t in a):
+                    return self.full(*args, **kwargs)
+        return self.light(*args, **kwargs)
+
+
+def _op(name, ns="mindpipe_amd"):
+    return lambda fn: _Op(fn, name, ns)
 
 
 # ---------------------------------------------------------------- W4
@@ -125,7 +180,7 @@ def unpack_int4(packed: torch.Tensor, k: int) -> torch.Tensor:
     return out
 
 
-@torch.library.custom_op("mindpipe_amd::w4a16_gemm", mutates_args=())
+@_op("w4a16_gemm")
 def w4a16_gemm(x: torch.Tensor, w_packed: torch.Tensor, scales: torch.Tensor, zeros: Optional[torch.Tensor],
                group_size: int, bias: Optional[torch.Tensor]) -> torch.Tensor:
     """``Y = X . dequant(W)^T (+ bias)``; ``x`` fp16 or bf16 ``[..., K]`` (scales, zeros, bias and
@@ -166,7 +221,7 @@ def _(x, w_packed, scales, zeros, group_size, bias):
 
 
 # ---------------------------------------------------------------- W8A8
-@torch.library.custom_op("mindpipe_amd::quant_per_token_i8", mutates_args=())
+@_op("quant_per_token_i8")
 def quant_per_token_i8(x: torch.Tensor, fake_rule: bool = False) -> Tuple[torch.Tensor, torch.Tensor]:
     """Per-token dynamic int8 quant: ``(q int8 [..., K], scale [...])``.
 
@@ -240,7 +295,7 @@ def add_rms_norm_quant(x: torch.Tensor, residual: Optional[torch.Tensor], weight
 # Functional custom ops over the fused norm (fixed output schemas, fake implementations), the form
 # torch.compile and graph capture take: the registration pattern of the reference's
 # torch.ops.vllm.* ops (vllm.patch:171-228,291-306).
-@torch.library.custom_op("mindpipe_amd::add_rms_norm_dynamic_quant", mutates_args=())
+@_op("add_rms_norm_dynamic_quant")
 def add_rms_norm_dynamic_quant(x: torch.Tensor, residual: torch.Tensor, weight: torch.Tensor,
                                eps: float) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
     """``(int8 codes, fp32 per-token scale, x + residual)`` of RMSNorm(x + residual) * weight
@@ -255,7 +310,7 @@ def _(x, residual, weight, eps):
             torch.empty(x.shape[:-1], dtype=torch.float32, device=x.device), torch.empty_like(x))
 
 
-@torch.library.custom_op("mindpipe_amd::rms_norm_dynamic_quant", mutates_args=())
+@_op("rms_norm_dynamic_quant")
 def rms_norm_dynamic_quant(x: torch.Tensor, weight: torch.Tensor, eps: float) -> Tuple[torch.Tensor, torch.Tensor]:
     """``(int8 codes, fp32 per-token scale)`` of RMSNorm(x) * weight (the first layer, no residual)."""
     _, q, sc, _ = add_rms_norm_quant(x, None, weight, eps, quant=True, out=False)
@@ -268,7 +323,7 @@ def _(x, weight, eps):
             torch.empty(x.shape[:-1], dtype=torch.float32, device=x.device))
 
 
-@torch.library.custom_op("mindpipe_amd::add_rms_norm", mutates_args=())
+@_op("add_rms_norm")
 def add_rms_norm(x: torch.Tensor, residual: torch.Tensor, weight: torch.Tensor,
                  eps: float) -> Tuple[torch.Tensor, torch.Tensor]:
     """``(RMSNorm(x + residual) * weight, x + residual)`` in x's dtype (``npu_add_rms_norm``)."""
@@ -307,7 +362,7 @@ def w8_quantize_per_channel(w: torch.Tensor, rule: str = "export"):
     return q, s32, ssrc
 
 
-@torch.library.custom_op("mindpipe_amd::w8a8_gemm", mutates_args=())
+@_op("w8a8_gemm")
 def w8a8_gemm(qx: torch.Tensor, s_tok: torch.Tensor, w: torch.Tensor, s_ch: torch.Tensor,
               bias: Optional[torch.Tensor], out_dtype: torch.dtype) -> torch.Tensor:
     """``((Qx . Qw^T) * s_tok) * s_ch (+ bias)`` -> ``out_dtype``; ``qx`` int8 ``[..., K]``, ``w`` int8 ``[N, K]``."""
@@ -342,7 +397,7 @@ def _(qx, s_tok, w, s_ch, bias, out_dtype):
     return qx.new_empty((*qx.shape[:-1], w.shape[0]), dtype=out_dtype)
 
 
-@torch.library.custom_op("mindpipe_amd::w8a8_gemm_fake", mutates_args=())
+@_op("w8a8_gemm_fake")
 def w8a8_gemm_fake(qx: torch.Tensor, s_tok: torch.Tensor, w: torch.Tensor, s_ch: torch.Tensor,
                    bias: Optional[torch.Tensor], act_dtype: torch.dtype) -> torch.Tensor:
     """``F.linear(r(qx * s_tok), r(w * s_ch), bias)`` in ``act_dtype`` (fp16 / bf16): the fake
@@ -377,8 +432,43 @@ def _(qx, s_tok, w, s_ch, bias, act_dtype):
     return qx.new_empty((*qx.shape[:-1], w.shape[0]), dtype=act_dtype)
 
 
-# in a namespace of its own: torch.ops.mindpipe_amd holds the reference's operator contracts
-@torch.library.custom_op("mindpipe_amd_fake::w8a8_linear", mutates_args=())
+# The linears from unquantized activations, in a namespace of their own: torch.ops.mindpipe_amd holds the reference's
+# operator contracts.
+@_op("w8a8_linear", "mindpipe_amd_fake")
+def w8a8_linear(x: torch.Tensor, w: torch.Tensor, s_ch: torch.Tensor, bias: Optional[torch.Tensor],
+                out_dtype: torch.dtype, fake_rule: bool) -> torch.Tensor:
+    """``quant_per_token_i8(x, fake_rule)`` then ``w8a8_gemm`` in one call, the same bits: the codes and fp32 scales
+    go through a workspace, with no scale conversion launch in between."""
+    _need(x, "x", (torch.float16, torch.bfloat16) if fake_rule else (torch.float16, torch.bfloat16, torch.float32))
+    _need(w, "w", torch.int8, 2)
+    _need(s_ch, "s_ch", torch.float32, 1)
+    k = x.shape[-1]
+    n = w.shape[0]
+    if w.shape[1] != k:
+        raise RuntimeError(f"weight {tuple(w.shape)} does not match K={k}")
+    if s_ch.numel() != n:
+        raise RuntimeError("scale sizes do not match M / N")
+    if bias is not None:
+        _need(bias, "bias", (torch.float16, torch.bfloat16, torch.float32), 1)
+    m = x.reshape(-1, k).shape[0]
+    y = torch.empty((*x.shape[:-1], n), dtype=out_dtype, device=x.device)
+    lib = _lib.load()
+    wsb = lib.mp_w8a8_linear_workspace_bytes(m, n, k)
+    ws = torch.empty((wsb,), dtype=torch.uint8, device=x.device)
+    with _dev(x):
+        _lib.check(lib.mp_w8a8_linear(
+            x.data_ptr(), _DT[x.dtype], m, k, w.data_ptr(), s_ch.data_ptr(), n, _ptr(bias),
+            _DT[bias.dtype] if bias is not None else MP_F16, y.data_ptr(), _DT[out_dtype],
+            MP_SCALE_FAKE if fake_rule else MP_SCALE_FP32, ws.data_ptr(), wsb, _stream()), "mp_w8a8_linear")
+    return y
+
+
+@w8a8_linear.register_fake
+def _(x, w, s_ch, bias, out_dtype, fake_rule):
+    return x.new_empty((*x.shape[:-1], w.shape[0]), dtype=out_dtype)
+
+
+@_op("w8a8_linear_fake", "mindpipe_amd_fake")
 def w8a8_linear_fake(x: torch.Tensor, w: torch.Tensor, s_ch: torch.Tensor,
                      bias: Optional[torch.Tensor]) -> torch.Tensor:
     """``F.linear(fake_quant(x), r(w * s_ch), bias)`` in ``x``'s dtype (fp16 / bf16): the per-token
@@ -464,7 +554,7 @@ def dq_linear(a: torch.Tensor, a_scale: Optional[torch.Tensor], b: torch.Tensor,
     return y.reshape(*a.shape[:-1], n)
 
 
-@torch.library.custom_op("mindpipe_amd::w8a8_gemm_quant_out", mutates_args=())
+@_op("w8a8_gemm_quant_out")
 def w8a8_gemm_quant_out(qx: torch.Tensor, s_tok: torch.Tensor, w: torch.Tensor, s_ch: torch.Tensor,
                         bias: Optional[torch.Tensor], out_dtype: torch.dtype,
                         fake_rule: bool = False) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
@@ -551,7 +641,7 @@ def moe_permute_quant(x: torch.Tensor, topk_ids: torch.Tensor, n_experts: int, r
     return routed, rscale, row_of_slot, offsets
 
 
-@torch.library.custom_op("mindpipe_amd::i8_gemm_swiglu_requant", mutates_args=())
+@_op("i8_gemm_swiglu_requant")
 def moe_gmm1_swiglu_quant(routed: torch.Tensor, rscale: torch.Tensor, w13: torch.Tensor, s13: torch.Tensor,
                           offsets: torch.Tensor, inter: int, rule: str = "runtime",
                           act_dtype: torch.dtype = torch.float16) -> Tuple[torch.Tensor, torch.Tensor]:
@@ -664,7 +754,7 @@ def _moe_fake(x, topk_ids, topk_w, w13, s13, w2, s2, out_dtype):
     return out
 
 
-@torch.library.custom_op("mindpipe_amd::moe_w8a8_forward", mutates_args=())
+@_op("moe_w8a8_forward")
 def moe_w8a8_forward(x: torch.Tensor, topk_ids: torch.Tensor, topk_w: torch.Tensor, w13: torch.Tensor,
                      s13: torch.Tensor, w2: torch.Tensor, s2: torch.Tensor, out_dtype: Optional[torch.dtype] = None,
                      rule: str = "runtime", x_scale: Optional[torch.Tensor] = None) -> torch.Tensor:
@@ -697,7 +787,7 @@ def _(x, topk_ids, topk_w, w13, s13, w2, s2, out_dtype=None, rule="runtime", x_s
     return x.new_empty((x.shape[0], w2.shape[1]), dtype=out_dtype)
 
 
-@torch.library.custom_op("mindpipe_amd::dense_mlp_w8a8", mutates_args=())
+@_op("dense_mlp_w8a8")
 def dense_mlp_w8a8(qx: torch.Tensor, sx: torch.Tensor, offsets: torch.Tensor, w13_chunks: List[torch.Tensor],
                    s13_chunks: List[torch.Tensor], w2_chunks: torch.Tensor, s2: torch.Tensor, chunk_size: int,
                    out_dtype: torch.dtype) -> torch.Tensor:

@@ -62,6 +62,9 @@ class W8A8DynamicLinearMethod:
             if x.dim() > 2:
                 output_shape = x.shape[:-1]
                 x = x.reshape(-1, x.shape[-1])
+            if config.get("pertoken_scale", True) and not config.get("return_scale", False):
+                output = ops.w8a8_linear(x.contiguous(), layer.weight, layer.weight_scale_fp32, bias, output_dtype, False)
+                return output if output_shape is None else output.reshape(*output_shape, output.shape[-1])
             quantized_x, dynamic_scale = dynamic_quant(x)
         else:
             output_dtype = config.get("output_dtype", getattr(layer, "params_dtype", torch.float16))

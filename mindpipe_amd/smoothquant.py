@@ -198,11 +198,15 @@ class SmoothQuantLinear(nn.Module):
             return self.output_quant(self._linear_any_width(x))
         if self._bf16_fake(x):
             return self.output_quant(self._linear_values(x))
+        fake = self.scale_rule == "fake"
+        if not self._fused_output_quant(x, fake):
+            if fake and x.dtype not in _FAKE_DTYPES:
+                raise NotImplementedError("the fake scale rule takes fp16 or bf16 activations")
+            return self.output_quant(ops.w8a8_linear(x.contiguous(), self.weight, self.weight_scale, self.bias, x.dtype,
+                                                     fake))
         fake, q, s = self._input_codes(x)
-        if self._fused_output_quant(x, fake):
-            qo, so = self._output_codes(q, s, x.dtype)
-            return (qo.float() * so.unsqueeze(-1)).to(x.dtype)
-        return self.output_quant(self._linear(x, fake, q, s))
+        qo, so = self._output_codes(q, s, x.dtype)
+        return (qo.float() * so.unsqueeze(-1)).to(x.dtype)
 
     def _input_codes(self, x):
         fake = self.scale_rule == "fake"

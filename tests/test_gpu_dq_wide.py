@@ -95,6 +95,6 @@ def test_linear_op_traces():
     gen = torch.Generator(device="cuda").manual_seed(3)
     q, s, _ = _weight((72, 128), torch.bfloat16, gen)
     x = torch.randn(2, 3, 128, generator=gen, device="cuda").bfloat16()
-    torch.library.opcheck(torch.ops.mindpipe_amd_fake.w8a8_linear.default, (x, q, s, None))
+    torch.library.opcheck(torch.ops.mindpipe_amd_fake.w8a8_linear_fake.default, (x, q, s, None))
     fn = torch.compile(lambda v: ops.w8a8_linear_fake(v, q, s, None), fullgraph=True, backend="aot_eager")
     assert torch.equal(fn(x), ops.w8a8_linear_fake(x, q, s, None))

@@ -82,6 +82,18 @@ def test_int8_linear_bits(out, m, n, k):
     assert torch.equal(ops.w8a8_gemm(q, st, w, sc, None, out), ((acc * st[:, None]) * sc[None]).to(out))
 
 
+@pytest.mark.parametrize("fake", [False, True])
+@pytest.mark.parametrize("shape", [(1,), (5, 7), (2, 100), (1500,)])
+def test_linear_from_activations_equals_the_two_ops(fake, shape):
+    gen = _gen(*shape, 7)
+    x = torch.randn(*shape, 256, generator=gen, device="cuda").half()
+    w = torch.randint(-127, 128, (264, 256), generator=gen, device="cuda", dtype=torch.int8)
+    sc, b = torch.rand(264, generator=gen, device="cuda") * 0.01, torch.randn(264, generator=gen, device="cuda").half()
+    q, s = ops.quant_per_token_i8(x, fake)
+    ref = ops.w8a8_gemm(q, s.float(), w, sc, b, torch.float16)
+    assert torch.equal(ops.w8a8_linear(x, w, sc, b, torch.float16, fake), ref)
+
+
 @pytest.mark.parametrize("t,e,top,h,inter", [(1, 64, 1, 128, 448), (48, 8, 2, 256, 3136), (700, 8, 2, 3200, 1536),
                                              (300, 2, 1, 12416, 12352), (64, 32, 4, 3072, 896)])
 def test_int8_experts_bits(t, e, top, h, inter):
@@ -109,3 +121,18 @@ def test_int8_experts_bits(t, e, top, h, inter):
         differ += int(((hh / (hh.abs().amax(-1, keepdim=True) / 127)).round().to(torch.int8) != q[a:b]).sum())
         assert torch.equal(((q[a:b].double() @ w2[i].double().T).float() * s[a:b, None]) * s2[i][None], y[a:b])
     assert differ <= 1e-3 * q.numel()
+
+
+def test_light_ops_refuse_what_the_custom_ops_refuse():
+    x = torch.randn(2, 128, device="cuda").half()
+    w = torch.randint(-127, 128, (64, 128), device="cuda", dtype=torch.int8)
+    sc = torch.ones(64, device="cuda")
+    y = ops.w8a8_linear(x.clone().requires_grad_(True), w, sc, None, torch.float16, True)
+    with pytest.raises(RuntimeError):
+        y.sum().backward()
+    with pytest.raises(RuntimeError, match="GPU"):
+        ops.quant_per_token_i8(x.cpu())
+    fn = torch.compile(lambda v: ops.w8a8_linear(v, w, sc, None, torch.float16, True), fullgraph=True, backend="aot_eager")
+    assert torch.equal(fn(x), ops.w8a8_linear(x, w, sc, None, torch.float16, True))
+    for op in (torch.ops.mindpipe_amd_light.quant_per_token_i8.default, torch.ops.mindpipe_amd.quant_per_token_i8.default):
+        torch.library.opcheck(op, (x, True))
