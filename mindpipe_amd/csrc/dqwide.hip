@@ -351,7 +351,7 @@ __global__ __launch_bounds__(512, 2) void dq_wide_kernel(mp_dq_args p, int n_slo
 
 template <int DT, int EPI, int TN>
 int wide_launch(const mp_dq_args &p, int splits, float *part, hipStream_t stream) {
-  const int64_t slots = mp_cdiv(p.rows, 256) + (p.offsets ? p.n_experts : 0);
+  const int64_t slots = wide_row_slots(p.rows, p.offsets ? p.n_experts : 1);
   const int64_t cols = mp_cdiv(mp_cdiv(p.n, EPI == MP_EPI_SWIGLU ? 64 * TN : 128 * TN), 8) * 8;
   if (slots * cols * splits > INT32_MAX) return MP_ERR_SHAPE;
   const void *fn = reinterpret_cast<const void *>(dq_wide_kernel<DT, EPI, TN>);

@@ -40,14 +40,14 @@ __device__ __forceinline__ bool i8w_rows(const mp_i8_args &p, int64_t slot, int6
 // gate rows and the BN / 2 matching up rows), a wave up to 4 x TN MFMA 32x32x32 tiles, row tiles 2 i + wm.  LDS:
 // three activation stages of K = 128 sized by the row tiles that are there, weight stages of K = 128 in the rest;
 // 128-byte rows, 16-byte chunk c of row r at slot c ^ ((r >> 1) & 7).  Waves 0..3 load the weights, 4..7 the activations,
-// and run one phase apart.  PART: split `part` of the K steps, int32 sums to p.y [splits, rows, n].
+// and run one phase apart.  SwiGLU with TN = 1: a wave's 32 weight rows are 16 gate rows and their up rows.  PART: split `part` of the K steps, int32 sums to p.y [splits, rows, n].
 template <int EPI, int TN, bool PART>
 __global__ __launch_bounds__(512, 2) void i8_wide_kernel(mp_i8_args p, int n_slots, int splits) {
   constexpr bool SWI = EPI == MP_EPI_SWIGLU;
   constexpr int TM = 4, WN = 4, BN = 128 * TN;
   constexpr int QB = BN / 8 / 4;
   constexpr int BST = BN * 128;
-  static_assert((!SWI || TN == 2) && !(SWI && PART), "forms");
+  static_assert(!(SWI && PART), "forms");
   extern __shared__ __attribute__((aligned(16))) int8_t smem_i8w[];
   int bx = static_cast<int>(blockIdx.x);
   int part = 0;
@@ -80,8 +80,10 @@ __global__ __launch_bounds__(512, 2) void i8_wide_kernel(mp_i8_args p, int n_slo
     if (wm == 1) {
       voff[q] = r < rows ? static_cast<uint32_t>(r) * k + ch : kWOob;
     } else {
-      const int c = c0 + (SWI ? r % (BN / 2) : r);
-      const uint32_t row = static_cast<uint32_t>(c + (SWI && r >= BN / 2 ? n_out : 0));
+      // SwiGLU: BN / 2 gate rows then their up rows, with one tile per wave 16 gate and 16 up rows by turns
+      const int c = c0 + (!SWI ? r : (TN == 2 ? r % (BN / 2) : r / 32 * 16 + r % 16));
+      const bool up = SWI && (TN == 2 ? r >= BN / 2 : r % 32 >= 16);
+      const uint32_t row = static_cast<uint32_t>(c + (up ? n_out : 0));
       voff[q] = c < n_out && r < BN ? row * k + ch : kWOob;
     }
   }
@@ -218,6 +220,59 @@ __global__ __launch_bounds__(512, 2) void i8_wide_kernel(mp_i8_args p, int n_slo
   const int esz = PART || SWI || EPI == MP_EPI_F32 || p.out_dtype == MP_F32 ? 4 : 2;
   const bool vec = n_out % 4 == 0 && p.ldy % 4 == 0 && (reinterpret_cast<uintptr_t>(p.y) & (4 * esz - 1)) == 0;
   const int64_t prow = PART ? part * p.rows : 0;
+  if constexpr (SWI && TN == 1) {
+    // a wave's tile is 16 gate columns and the matching 16 up columns: the products meet in the staged tile, a lane
+    // then holds two output columns of a row; the abs-max of 32 columns joins two waves' in LDS
+    float *samax = stok + 256;  // [256 rows][4 wave columns]
+    const int cw0 = c0 + wn * 16, cl = min(cw0 + (lane & 15), n_out - 1);
+    const float sc = sbx[((lane & 16) ? n_out : 0) + cl];
+    const bool pair = n_out % 2 == 0 && p.ldy % 2 == 0 && (reinterpret_cast<uintptr_t>(p.y) & 7) == 0;
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+      if (i >= nv) continue;  // wave-uniform
+      const int lr = (i * 2 + wm) * 32;
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const f4_t st4 = *reinterpret_cast<const f4_t *>(stok + lr + 8 * g + 4 * half);
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          *reinterpret_cast<float *>(stage + (8 * g + 4 * half + e) * LDR + (lane & 31) * 4) =
+              mp_mul(mp_mul(static_cast<float>(acc[i][0][4 * g + e]), st4[e]), sc);
+      }
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int row = q * 8 + lane / 8, col = cw0 + (lane & 7) * 2;
+        const int64_t m = rb + lr + row, o = m * p.ldy + col;
+        float a = 0.f, h[2];
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          const float *gu = reinterpret_cast<const float *>(stage + row * LDR) + (lane & 7) * 2 + e;
+          h[e] = mp_swiglu_epi(gu[0], gu[16], p.epi_round);
+          if (col + e < n_out) a = fmaxf(a, fabsf(h[e]));
+        }
+        a = fmaxf(a, __shfl_xor(a, 1, 64));
+        a = fmaxf(a, __shfl_xor(a, 2, 64));
+        a = fmaxf(a, __shfl_xor(a, 4, 64));
+        if ((lane & 7) == 0) samax[(lr + row) * 4 + wn] = a;
+        if (m >= re) continue;
+        float *yo = reinterpret_cast<float *>(yb) + o;
+        if (pair) {
+          if (col < n_out) *reinterpret_cast<float2 *>(yo) = make_float2(h[0], h[1]);
+        } else {
+#pragma unroll
+          for (int e = 0; e < 2; ++e)
+            if (col + e < n_out) yo[e] = h[e];
+        }
+      }
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the next tile overwrites the region
+    }
+    mp_lds_barrier();
+    const int row = tid / 2, w = (tid & 1) * 2;
+    if (row < rows && c0 / 32 + (tid & 1) < p.n_partial)
+      p.amax_partial[(rb + row) * p.n_partial + c0 / 32 + (tid & 1)] = fmaxf(samax[row * 4 + w], samax[row * 4 + w + 1]);
+    return;
+  }
   if constexpr (EPI == MP_EPI_DENSE && !PART) {
     // 16-bit outputs in whole 16-byte chunks: the wave's columns of a row tile staged as 16-bit values (row stride
     // 64 TN + 16 bytes), so that a row of the wave is one 64 TN byte segment of memory, in 16-byte stores (M = 4096,
@@ -371,7 +426,7 @@ __global__ __launch_bounds__(256) void i8_reduce_kernel(const int *__restrict__ 
 
 template <int EPI, int TN, bool PART>
 int i8w_launch(const mp_i8_args &p, int splits, hipStream_t stream) {
-  const int64_t slots = mp_cdiv(p.rows, 256) + (p.offsets ? p.n_experts : 0);
+  const int64_t slots = wide_row_slots(p.rows, p.offsets ? p.n_experts : 1);
   const int64_t cols = mp_cdiv(mp_cdiv(p.n, EPI == MP_EPI_SWIGLU ? 64 * TN : 128 * TN), 8) * 8;
   if (slots * cols * splits > INT32_MAX) return MP_ERR_SHAPE;
   const void *fn = reinterpret_cast<const void *>(i8_wide_kernel<EPI, TN, PART>);
@@ -391,11 +446,12 @@ bool mp_i8_wide_takes(const mp_i8_args &p, int epi) {
 }
 
 int mp_launch_i8_wide(const mp_i8_args &p, int epi, hipStream_t stream) {
-  if (epi == MP_EPI_SWIGLU) return i8w_launch<MP_EPI_SWIGLU, 2, false>(p, 1, stream);
   const int64_t cus = mp_cu_count() > 0 ? mp_cu_count() : 256;
   const int64_t groups = p.offsets ? (p.rows < p.n_experts ? p.rows : p.n_experts) : 1;
-  const int64_t tiles = mp_cdiv(p.n, 256) * groups * mp_cdiv(mp_cdiv(p.rows, groups), 256);
+  const int64_t tiles = mp_cdiv(epi == MP_EPI_SWIGLU ? 2 * p.n : p.n, 256) * groups * mp_cdiv(mp_cdiv(p.rows, groups), 256);
   const bool two = 4 * tiles >= 3 * cus;  // 256 weight rows per workgroup, see wide_pick (dqwide.hip)
+  if (epi == MP_EPI_SWIGLU)
+    return two ? i8w_launch<MP_EPI_SWIGLU, 2, false>(p, 1, stream) : i8w_launch<MP_EPI_SWIGLU, 1, false>(p, 1, stream);
   if (epi == MP_EPI_F32) return two ? i8w_launch<MP_EPI_F32, 2, false>(p, 1, stream) : i8w_launch<MP_EPI_F32, 1, false>(p, 1, stream);
   return two ? i8w_launch<MP_EPI_DENSE, 2, false>(p, 1, stream) : i8w_launch<MP_EPI_DENSE, 1, false>(p, 1, stream);
 }

@@ -2187,14 +2187,18 @@ static int mp_launch_moe(const mp_i8_args &a, hipStream_t stream) {
 //   run: M = 800, 8192 x 8192 86 against 109 us, M = 512, N = 11008 46 against 54 us, M = 64, N = 11008 / 28672 26.5 / 35
 //   against 31 / 44 us (the mid-M kernel's smaller tiles win at M = 256, N = 11008: 29 against 39 us);
 //   grouped, from three tiles for four CUs, against i8_moe_kernel: the Mixtral-shaped chain at 4 / 16 / 48 / 512 /
-//   1000 tokens 227 / 306 / 309 / 412 / 667 against 283 / 337 / 344 / 457 / 744 us (one group of 200 rows, I = 11008: 86
-//   tiles, GEMM1 63 against 46 us).
+//   1000 tokens 227 / 306 / 309 / 412 / 667 against 283 / 337 / 344 / 457 / 744 us;
+//   SwiGLU at every size (64 output columns per workgroup where 128 would not fill the CUs): the dense MLP chain
+//   (4096, I = 11008) at 2 / 16 / 96 / 200 / 256 / 400 rows 52 / 53 / 72 / 86 / 91 / 132 against 61 / 62 / 78 / 88 / 94 /
+//   175 us, the expert chain of eight experts (2048, I = 1408) at 8 / 64 / 512 tokens 46 / 49 / 69 against 51 / 52 / 71.
 static bool mp_wide_takes(const mp_i8_args &a, int epilogue) {
   if (epilogue == MP_EPI_AMAX || !mp_i8_wide_takes(a, epilogue)) return false;
   const int64_t cus = mp_cu_count() > 0 ? mp_cu_count() : 256;
+  if (epilogue == MP_EPI_SWIGLU) return true;
   if (a.offsets) {
     const int64_t groups = a.rows < a.n_experts ? a.rows : a.n_experts;
-    return 4 * mp_cdiv(a.n, 128) * groups * mp_cdiv(mp_cdiv(a.rows, groups), 256) >= 3 * cus;
+    const int64_t chunks = groups * mp_cdiv(mp_cdiv(a.rows, groups), 256);
+    return 4 * mp_cdiv(a.n, 128) * chunks >= 3 * cus;
   }
   if (epilogue != MP_EPI_DENSE || a.rows <= 32) return false;
   if (a.rows >= 1024) return true;

@@ -95,7 +95,9 @@ def test_linear_from_activations_equals_the_two_ops(fake, shape):
 
 
 @pytest.mark.parametrize("t,e,top,h,inter", [(1, 64, 1, 128, 448), (48, 8, 2, 256, 3136), (700, 8, 2, 3200, 1536),
-                                             (300, 2, 1, 12416, 12352), (64, 32, 4, 3072, 896)])
+                                             (300, 2, 1, 12416, 12352), (64, 32, 4, 3072, 896),
+                                             # 64 output columns per workgroup: one group, few tiles, several chunks
+                                             (1, 1, 1, 128, 64), (33, 1, 1, 256, 192), (257, 1, 1, 384, 1088), (513, 3, 2, 256, 320)])
 def test_int8_experts_bits(t, e, top, h, inter):
     """GEMM1 + SwiGLU + requant and GEMM2 over groups of 0 to 350 rows: GEMM2 bit for bit; the codes up to those that
     exp's last bit decides."""
