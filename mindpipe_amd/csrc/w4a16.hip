@@ -560,6 +560,15 @@ __global__ __launch_bounds__(S * 64) void w4a16_batch_kernel(
   const int st_lo = (nst * wave) / S;
   const int nsteps = (nst * (wave + 1)) / S - st_lo;
   const int lo = st_lo * STEP;
+  // One wave per workgroup walks the whole of K: workgroups start at different steps of it, or all would read the
+  // same column window of the weight rows at a time, which with a power-of-two row is a few memory channels (16 rows
+  // of K = 8192 at N = 128256: 138 -> 129 us, at N = 57344: 72 -> 68 us).  Waves that split K are spread already
+  // (all shapes within 1%, so they keep the plain order).
+  const int rot = S == 1 ? bx % nsteps : 0;
+  auto at = [&](int st) {  // first block of the st-th step taken
+    const int q = st + rot;
+    return lo + (S > 1 || q < nsteps ? q : q - nsteps) * STEP;
+  };
   uint32_t magic_v = kMagic, mask_v = 0x000F000Fu, mask1_v = 0x00F000F0u;
   asm volatile("" : "+v"(magic_v), "+v"(mask_v), "+v"(mask1_v));
   const h8_t ones = {1, 1, 1, 1, 1, 1, 1, 1};
@@ -719,11 +728,11 @@ __global__ __launch_bounds__(S * 64) void w4a16_batch_kernel(
     // activations one pair ahead in two buffers, the next step's scales during the
     // current step's last pair (its words copied out first): a pair waits only for loads
     // issued a pair or more before it
-    issue_w(wa, lo);
-    load_x_to(xa, lo);
-    load_sz(lo);
+    issue_w(wa, at(0));
+    load_x_to(xa, at(0));
+    load_sz(at(0));
     for (int st = 0; st < nsteps; ++st) {
-      const int b = lo + st * STEP;
+      const int b = at(st);
       uint32_t swd[NT], zwd[NT];
       load_x_to(xb, b + 2);
       issue_w(wb, b + 2);
@@ -744,7 +753,7 @@ __global__ __launch_bounds__(S * 64) void w4a16_batch_kernel(
       compute_x(wa, xa, swd, zwd);
       __builtin_amdgcn_sched_barrier(0);
       words(3, swd, zwd);
-      const int nb = st + 1 < nsteps ? b + STEP : nblk;  // past the range: reads nothing
+      const int nb = st + 1 < nsteps ? at(st + 1) : nblk;  // past the range: reads nothing
       load_x_to(xa, nb);
       issue_w(wa, nb);
       load_sz(nb);
@@ -753,9 +762,9 @@ __global__ __launch_bounds__(S * 64) void w4a16_batch_kernel(
       __builtin_amdgcn_sched_barrier(0);
     }
   } else {
-  issue_w(wa, lo);
+  issue_w(wa, at(0));
   for (int st = 0; st < nsteps; ++st) {
-    const int b = lo + st * STEP;
+    const int b = at(st);
     load_sz(b);
     load_x(b);
     __builtin_amdgcn_sched_barrier(0);
@@ -777,7 +786,7 @@ __global__ __launch_bounds__(S * 64) void w4a16_batch_kernel(
     __builtin_amdgcn_sched_barrier(0);
     load_x(b + 6);
     __builtin_amdgcn_sched_barrier(0);
-    issue_w(wa, st + 1 < nsteps ? b + STEP : nblk);  // the last prefetch reads nothing
+    issue_w(wa, st + 1 < nsteps ? at(st + 1) : nblk);  // the last prefetch reads nothing
     __builtin_amdgcn_sched_barrier(0);
     compute(wb, 3);
     __builtin_amdgcn_sched_barrier(0);
