@@ -141,7 +141,7 @@ int wide_reduce(const float *part, int splits, int64_t m, int64_t n, const void 
 
 // Row slots of 256 that hold any split of `rows` into `groups` groups: sum ceil(r / 256) <= (rows + 255 groups) / 256.
 // No more than that: workgroups go to the shader engines by turns, and a single group's spare slot (every other
-// workgroup empty) left half of the engines idle (200 rows, 11008 gate / up pairs x 4096: 74 -> 39 us).
+// workgroup empty) left half of the engines idle (200 rows, 11008 gate / up pairs x 4096: 74 -> 43 us).
 static inline int64_t wide_row_slots(int64_t rows, int64_t groups) {
   return (rows + 255 * (groups < rows ? groups : rows)) / 256;
 }

@@ -125,6 +125,24 @@ def test_int8_experts_bits(t, e, top, h, inter):
     assert differ <= 1e-3 * q.numel()
 
 
+@pytest.mark.parametrize("rows,inter", [(1, 63), (3, 1027), (2, 2052), (300, 1030), (2049, 260)])
+def test_gate_up_columns(rows, inter):
+    """Column counts that vector accesses and the requant's column parts do not divide; codes up to exp's last bit."""
+    gen = _gen(rows, inter)
+    x = torch.randint(-127, 128, (rows, 256), generator=gen, device="cuda", dtype=torch.int8)
+    rs = torch.rand(rows, generator=gen, device="cuda") * 0.01 + 1e-3
+    w = torch.randint(-127, 128, (1, 2 * inter, 256), generator=gen, device="cuda", dtype=torch.int8)
+    sc = torch.rand(1, 2 * inter, generator=gen, device="cuda") * 1e-3
+    off = torch.tensor([0, rows], device="cuda", dtype=torch.int64)
+    q, s = ops.moe_gmm1_swiglu_quant(x, rs, w, sc, off, inter)
+    gu = ((x.double() @ w[0].double().T).float() * rs[:, None]) * sc
+    hh = gu[:, :inter] / (1 + torch.exp(-gu[:, :inter])) * gu[:, inter:]
+    amax = hh.abs().amax(-1)
+    assert torch.allclose(s.view(-1), amax / 127, rtol=1e-5)
+    diff = ((hh / (amax[:, None] / 127)).round().int() - q.int()).abs()
+    assert int(diff.max()) <= 1 and int((diff != 0).sum()) <= max(1, 1e-3 * q.numel())
+
+
 def test_light_ops_refuse_what_the_custom_ops_refuse():
     x = torch.randn(2, 128, device="cuda").half()
     w = torch.randint(-127, 128, (64, 128), device="cuda", dtype=torch.int8)
