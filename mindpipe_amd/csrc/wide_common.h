@@ -1,4 +1,4 @@
-// Device helpers of the direct-to-LDS GEMMs (dqwide.hip, w4wide.hip).
+// Device helpers of the direct-to-LDS GEMMs (dqwide.hip, i8wide.hip, w4wide.hip).
 #pragma once
 #include "mp_common.h"
 
