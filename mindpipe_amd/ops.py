@@ -63,42 +63,41 @@ def _dev(t: torch.Tensor):
 _LIGHT = torch.library.Library("mindpipe_amd_light", "DEF")
 
 
-class _Op:
-    """An op registered twice over one function: as the custom op ``torch.ops.mindpipe_amd.<name>`` and, without that
-    wrapper's Python autograd layer, as ``torch.ops.mindpipe_amd_light.<name>`` with the same fake implementation.
-    A call goes to the custom op under compilation, functorch transforms and forward-mode AD and where an
-    input requires a gradient (it refuses the backward); otherwise to the light one: the custom op's layers cost
-    about 11 us a call, half of an eager one-row linear (23 us)."""
-
-    def __init__(self, fn, name, ns):
-        self.fn, self.name, self.__doc__, self.__name__ = fn, name, fn.__doc__, fn.__name__
-        self.def_ = torch.library.custom_op(f"{ns}::{name}", mutates_args=())(fn)
-        _LIGHT.define(name + torch.library.infer_schema(fn, mutates_args=()))
-        _LIGHT.impl(name, fn, "CompositeExplicitAutograd")
-        self.full = getattr(getattr(torch.ops, ns), name).default
-        self.light = getattr(torch.ops.mindpipe_amd_light, name).default
+class _Op(torch.library.CustomOpDef):
+    """The custom op ``torch.ops.<ns>.<name>``, whose eager calls go to ``torch.ops.mindpipe_amd_light.<name>``: the same
+    function and fake implementation without the custom op's Python autograd layer.  A call goes to the custom op
+    itself under compilation, functorch transforms and forward-mode AD and where an input requires a gradient (it
+    refuses the backward); its layers cost about 11 us a call, half of an eager one-row linear (23 us)."""
 
     def register_fake(self, fake):
-        self.def_.register_fake(fake)
-        torch.library.register_fake(f"mindpipe_amd_light::{self.name}", fake, lib=_LIGHT)
+        super().register_fake(fake)
+        torch.library.register_fake(f"mindpipe_amd_light::{self.light_name}", fake, lib=_LIGHT)
         return fake
 
     def __call__(self, *args, **kwargs):
         if (torch.compiler.is_compiling() or torch._C._functorch.peek_interpreter_stack() is not None
                 or torch.autograd.forward_ad._current_level >= 0):
-            return self.full(*args, **kwargs)
+            return super().__call__(*args, **kwargs)
         if torch.is_grad_enabled():
             for a in (*args, *kwargs.values()):
                 if isinstance(a, torch.Tensor):
                     if a.requires_grad:
-                        return self.full(*args, **kwargs)
+                        return super().__call__(*args, **kwargs)
                 elif isinstance(a, (list, tuple)) and any(isinstance(t, torch.Tensor) and t.requires_grad for t in a):
-                    return self.full(*args, **kwargs)
+                    return super().__call__(*args, **kwargs)
         return self.light(*args, **kwargs)
 
 
 def _op(name, ns="mindpipe_amd"):
-    return lambda fn: _Op(fn, name, ns)
+    def register(fn):
+        op = torch.library.custom_op(f"{ns}::{name}", mutates_args=())(fn)
+        op.__class__ = _Op  # torch.library.custom_op is the only way to make a CustomOpDef
+        op.light_name, op.__name__, op.__doc__ = name, fn.__name__, fn.__doc__
+        _LIGHT.define(name + torch.library.infer_schema(fn, mutates_args=()))
+        _LIGHT.impl(name, fn, "CompositeExplicitAutograd")
+        op.light = getattr(torch.ops.mindpipe_amd_light, name).default
+        return op
+    return register
 
 
 # ---------------------------------------------------------------- W4
