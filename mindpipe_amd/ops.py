@@ -61,13 +61,27 @@ def _dev(t: torch.Tensor):
 
 # ---------------------------------------------------------------- registration
 _LIGHT = torch.library.Library("mindpipe_amd_light", "DEF")
+_PLAIN = (torch.Tensor, torch.nn.Parameter)
+_IMPLS = torch.library._impls  # "ns/op/key" of every torch.library.impl
 
 
 class _Op(torch.library.CustomOpDef):
     """The custom op ``torch.ops.<ns>.<name>``, whose eager calls go to ``torch.ops.mindpipe_amd_light.<name>``: the same
     function and fake implementation without the custom op's Python autograd layer.  A call goes to the custom op
     itself under compilation, functorch transforms and forward-mode AD and where an input requires a gradient (it
-    refuses the backward); its layers cost about 11 us a call, half of an eager one-row linear (23 us)."""
+    refuses the backward); its layers cost about 11 us a call, half of an eager one-row linear (23 us).  So does
+    every call without a plain CUDA tensor and, once a kernel or autocast rule is registered for it, every call:
+    the light op knows only this package's kernels."""
+
+    registered = False  # the user's kernel or autocast rule stands in the custom op
+
+    def register_kernel(self, *args, **kwargs):
+        self.registered = True
+        return super().register_kernel(*args, **kwargs)
+
+    def register_autocast(self, *args, **kwargs):
+        self.registered = True
+        return super().register_autocast(*args, **kwargs)
 
     def register_fake(self, fake):
         super().register_fake(fake)
@@ -75,15 +89,14 @@ class _Op(torch.library.CustomOpDef):
         return fake
 
     def __call__(self, *args, **kwargs):
-        if (torch.compiler.is_compiling() or torch._C._functorch.peek_interpreter_stack() is not None
+        if (self.registered or self.cuda_impl in _IMPLS or torch.compiler.is_compiling()
+                or torch._C._functorch.peek_interpreter_stack() is not None
                 or torch.autograd.forward_ad._current_level >= 0):
             return super().__call__(*args, **kwargs)
-        if torch.is_grad_enabled():
-            for a in (*args, *kwargs.values()):
-                if isinstance(a, torch.Tensor):
-                    if a.requires_grad:
-                        return super().__call__(*args, **kwargs)
-                elif isinstance(a, (list, tuple)) and any(isinstance(t, torch.Tensor) and t.requires_grad for t in a):
+        grad = torch.is_grad_enabled()
+        for a in (*args, *kwargs.values()):
+            for t in (a,) if isinstance(a, torch.Tensor) else a if isinstance(a, (list, tuple)) else ():
+                if type(t) not in _PLAIN or not t.is_cuda or (grad and t.requires_grad):
                     return super().__call__(*args, **kwargs)
         return self.light(*args, **kwargs)
 
@@ -92,6 +105,7 @@ def _op(name, ns="mindpipe_amd"):
     def register(fn):
         op = torch.library.custom_op(f"{ns}::{name}", mutates_args=())(fn)
         op.__class__ = _Op  # torch.library.custom_op is the only way to make a CustomOpDef
+        op.cuda_impl = f"{ns}/{name}/CUDA"
         op.light_name, op.__name__, op.__doc__ = name, fn.__name__, fn.__doc__
         _LIGHT.define(name + torch.library.infer_schema(fn, mutates_args=()))
         _LIGHT.impl(name, fn, "CompositeExplicitAutograd")

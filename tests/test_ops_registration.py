@@ -1,11 +1,16 @@
 """What torch's public registration and tracing APIs see of the operators, on the CPU."""
 import inspect
+import subprocess
+import sys
+import textwrap
+from pathlib import Path
 
 import pytest
 import torch
 
 from mindpipe_amd import ops
 
+ROOT = Path(__file__).resolve().parent.parent
 OPS = [n for n in dir(ops) if isinstance(getattr(ops, n), torch.library.CustomOpDef)]
 
 
@@ -19,3 +24,38 @@ def test_every_registered_op_is_a_custom_op_def():
 def test_custom_op_def_methods(name):
     method = getattr(ops.w4a16_gemm, name)
     assert callable(method) and inspect.signature(method)
+
+
+def _python(code):
+    """Runs ``code`` in a process of its own: registrations and reloads outlive a test."""
+    head = "import importlib, torch\nfrom mindpipe_amd import ops\nx = torch.randn(2, 64).half()\n"
+    subprocess.run([sys.executable, "-c", head + textwrap.dedent(code)], check=True, cwd=ROOT, timeout=120)
+
+
+@pytest.mark.parametrize("register", [
+    'torch.library.register_kernel("mindpipe_amd::quant_per_token_i8", "cpu", mine)',
+    'ops.quant_per_token_i8.register_kernel("cpu")(mine)',
+    'lib = torch.library.Library("mindpipe_amd", "IMPL"); lib.impl("quant_per_token_i8", mine, "CPU")',
+])
+def test_a_registered_kernel_is_used(register):
+    _python(f"""
+        mine = lambda v, fake_rule=False: (torch.zeros_like(v, dtype=torch.int8), torch.full((len(v),), 3.0))
+        {register}
+        for got in (ops.quant_per_token_i8(x), torch.ops.mindpipe_amd.quant_per_token_i8(x)):
+            assert got[1].tolist() == [3.0, 3.0]
+    """)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("register", [
+    'torch.library.register_kernel("mindpipe_amd::quant_per_token_i8", "cuda", mine)',
+    'lib = torch.library.Library("mindpipe_amd", "IMPL"); lib.impl("quant_per_token_i8", mine, "CUDA")',
+])
+def test_a_registered_gpu_kernel_is_used(register):
+    _python(f"""
+        x = x.cuda()
+        assert ops.quant_per_token_i8(x)[1].tolist() != [3.0, 3.0]
+        mine = lambda v, fake_rule=False: (torch.zeros_like(v, dtype=torch.int8), v.new_full((len(v),), 3.0))
+        {register}
+        assert ops.quant_per_token_i8(x)[1].tolist() == [3.0, 3.0]
+    """)
