@@ -60,6 +60,7 @@ def _dev(t: torch.Tensor):
 
 
 # ---------------------------------------------------------------- registration
+globals().pop("_LIGHT", None)  # of an earlier import: a reload defines the operators again
 _LIGHT = torch.library.Library("mindpipe_amd_light", "DEF")
 _PLAIN = (torch.Tensor, torch.nn.Parameter)
 _IMPLS = torch.library._impls  # "ns/op/key" of every torch.library.impl

@@ -46,6 +46,23 @@ def test_a_registered_kernel_is_used(register):
     """)
 
 
+def test_reload():
+    _python("""
+        old = ops.quant_per_token_i8
+        for _ in range(2):
+            importlib.reload(ops)
+        for op in (old, ops.quant_per_token_i8, torch.ops.mindpipe_amd.quant_per_token_i8):
+            try:
+                op(x)
+            except RuntimeError as e:
+                assert "must be on the GPU" in str(e)
+            else:
+                raise AssertionError("no CPU path")
+        y = torch.ops.mindpipe_amd_light.quant_per_token_i8(x.to("meta"), False)
+        assert y[0].shape == x.shape and y[0].is_meta
+    """)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("register", [
     'torch.library.register_kernel("mindpipe_amd::quant_per_token_i8", "cuda", mine)',
