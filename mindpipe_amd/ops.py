@@ -69,8 +69,8 @@ _IMPLS = torch.library._impls  # "ns/op/key" of every torch.library.impl
 class _Op(torch.library.CustomOpDef):
     """The custom op ``torch.ops.<ns>.<name>``, whose eager calls go to ``torch.ops.mindpipe_amd_light.<name>``: the same
     function and fake implementation without the custom op's Python autograd layer.  A call goes to the custom op
-    itself under compilation, functorch transforms and forward-mode AD and where an input requires a gradient (it
-    refuses the backward); its layers cost about 11 us a call, half of an eager one-row linear (23 us).  So does
+    itself under compilation, tracing, dispatch and function modes, functorch transforms and forward-mode AD and where
+    an input requires a gradient (it refuses the backward); its layers cost about 11 us a call, half of an eager one-row linear (23 us).  So does
     every call without a plain CUDA tensor and, once a kernel or autocast rule is registered for it, every call:
     the light op knows only this package's kernels."""
 
@@ -92,7 +92,8 @@ class _Op(torch.library.CustomOpDef):
     def __call__(self, *args, **kwargs):
         if (self.registered or self.cuda_impl in _IMPLS or torch.compiler.is_compiling()
                 or torch._C._functorch.peek_interpreter_stack() is not None
-                or torch.autograd.forward_ad._current_level >= 0):
+                or torch.autograd.forward_ad._current_level >= 0 or torch._C._len_torch_dispatch_stack()
+                or torch._C._len_torch_function_stack() or torch._C._get_tracing_state() is not None):
             return super().__call__(*args, **kwargs)
         grad = torch.is_grad_enabled()
         for a in (*args, *kwargs.values()):

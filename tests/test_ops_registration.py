@@ -1,4 +1,5 @@
 """What torch's public registration and tracing APIs see of the operators, on the CPU."""
+import concurrent.futures
 import inspect
 import subprocess
 import sys
@@ -76,3 +77,70 @@ def test_a_registered_gpu_kernel_is_used(register):
         {register}
         assert ops.quant_per_token_i8(x)[1].tolist() == [3.0, 3.0]
     """)
+
+
+@pytest.mark.gpu
+def test_traces_and_modes_see_the_custom_op():
+    from torch.fx.experimental.proxy_tensor import make_fx
+    from torch.overrides import TorchFunctionMode
+    from torch.utils._python_dispatch import TorchDispatchMode
+    x = torch.randn(2, 64, device="cuda").half()
+    graph = make_fx(lambda v: ops.quant_per_token_i8(v))(x).graph
+    assert torch.ops.mindpipe_amd.quant_per_token_i8.default in [n.target for n in graph.nodes]
+    seen = []
+
+    class Dispatch(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            seen.append(func)
+            return func(*args, **(kwargs or {}))
+
+    class Function(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            seen.append(func)
+            return func(*args, **(kwargs or {}))
+
+    for mode in (Dispatch, Function):
+        seen.clear()
+        with mode():
+            ops.quant_per_token_i8(x)
+        assert torch.ops.mindpipe_amd.quant_per_token_i8.default in seen
+
+
+def _outcome(f):
+    try:
+        return f()
+    except Exception as e:
+        return type(e)
+
+
+@pytest.mark.gpu
+def test_vmap_and_forward_ad_do_what_the_custom_op_does():
+    x = torch.randn(3, 2, 64, device="cuda").half()
+    direct, custom = ops.quant_per_token_i8, torch.ops.mindpipe_amd.quant_per_token_i8.default
+    got, want = (_outcome(lambda: torch.vmap(lambda v: op(v)[0])(x)) for op in (direct, custom))
+    assert torch.equal(got, want) if isinstance(want, torch.Tensor) else got == want
+    with torch.autograd.forward_ad.dual_level():
+        dual = torch.autograd.forward_ad.make_dual(x, torch.ones_like(x))
+        got, want = (_outcome(lambda: torch.autograd.forward_ad.unpack_dual(op(dual)[1]).tangent is None)
+                     for op in (direct, custom))
+        assert got == want
+
+
+@pytest.mark.gpu
+def test_other_streams_and_threads():
+    """Each stream and each thread's calls read and write on their own current stream."""
+    w = torch.randint(-127, 128, (512, 1024), device="cuda", dtype=torch.int8)
+    sc = torch.rand(512, device="cuda") * 0.01
+    xs = [torch.randn(64, 1024, device="cuda").half() for _ in range(4)]
+    want = [ops.w8a8_linear(x, w, sc, None, torch.float16, False) for x in xs]
+    torch.cuda.synchronize()
+
+    def work(x):
+        side = torch.cuda.Stream()
+        with torch.cuda.stream(side):
+            out = [ops.w8a8_linear(x, w, sc, None, torch.float16, False) for _ in range(20)]
+        side.synchronize()
+        return out
+    with concurrent.futures.ThreadPoolExecutor(4) as pool:
+        for got, ref in zip(pool.map(work, xs), want):
+            assert all(torch.equal(g, ref) for g in got)
