@@ -221,9 +221,9 @@ def w4a16_gemm(x: torch.Tensor, w_packed: torch.Tensor, scales: torch.Tensor, ze
     m = x2.shape[0]
     y = torch.empty((m, n), dtype=x.dtype, device=x.device)
     lib = _lib.load()
-    wsb = lib.mp_w4a16_gemm_workspace_bytes(m, n, k, group_size) if m > 32 else 0
-    ws = torch.empty((wsb,), dtype=torch.uint8, device=x.device) if wsb else None
-    with _dev(x):
+    with _dev(x):  # the K split, and so the workspace, goes by this device's CUs
+        wsb = lib.mp_w4a16_gemm_workspace_bytes(m, n, k, group_size) if m > 32 else 0
+        ws = torch.empty((wsb,), dtype=torch.uint8, device=x.device) if wsb else None
         _lib.check(lib.mp_w4a16_gemm_ws(
             x2.data_ptr(), m, k, w_packed.data_ptr(), n, scales.data_ptr(), _ptr(zeros), group_size,
             _ptr(bias), y.data_ptr(), _DT[x.dtype], _ptr(ws), wsb, _stream()), "mp_w4a16_gemm_ws")
@@ -397,9 +397,9 @@ def w8a8_gemm(qx: torch.Tensor, s_tok: torch.Tensor, w: torch.Tensor, s_ch: torc
         _need(bias, "bias", (torch.float16, torch.bfloat16, torch.float32), 1)
     y = torch.empty((m, n), dtype=out_dtype, device=qx.device)
     lib = _lib.load()
-    wsb = lib.mp_w8a8_gemm_workspace_bytes(m, n, k)
-    ws = torch.empty((wsb,), dtype=torch.uint8, device=qx.device) if wsb else None
     with _dev(qx):
+        wsb = lib.mp_w8a8_gemm_workspace_bytes(m, n, k)
+        ws = torch.empty((wsb,), dtype=torch.uint8, device=qx.device) if wsb else None
         _lib.check(lib.mp_w8a8_gemm_ws(
             q2.data_ptr(), s_tok.data_ptr(), w.data_ptr(), s_ch.data_ptr(), _ptr(bias),
             _DT[bias.dtype] if bias is not None else MP_F16, y.data_ptr(), _DT[out_dtype], m, n, k, _ptr(ws), wsb,
@@ -468,9 +468,9 @@ def w8a8_linear(x: torch.Tensor, w: torch.Tensor, s_ch: torch.Tensor, bias: Opti
     m = x.reshape(-1, k).shape[0]
     y = torch.empty((*x.shape[:-1], n), dtype=out_dtype, device=x.device)
     lib = _lib.load()
-    wsb = lib.mp_w8a8_linear_workspace_bytes(m, n, k)
-    ws = torch.empty((wsb,), dtype=torch.uint8, device=x.device)
     with _dev(x):
+        wsb = lib.mp_w8a8_linear_workspace_bytes(m, n, k)
+        ws = torch.empty((wsb,), dtype=torch.uint8, device=x.device)
         _lib.check(lib.mp_w8a8_linear(
             x.data_ptr(), _DT[x.dtype], m, k, w.data_ptr(), s_ch.data_ptr(), n, _ptr(bias),
             _DT[bias.dtype] if bias is not None else MP_F16, y.data_ptr(), _DT[out_dtype],
@@ -504,9 +504,9 @@ def w8a8_linear_fake(x: torch.Tensor, w: torch.Tensor, s_ch: torch.Tensor,
     m = x2.shape[0]
     y = torch.empty((*x.shape[:-1], n), dtype=x.dtype, device=x.device)
     lib = _lib.load()
-    wsb = lib.mp_w8a8_linear_fake_workspace_bytes(m, n, k)
-    ws = torch.empty((wsb,), dtype=torch.uint8, device=x.device)
     with _dev(x):
+        wsb = lib.mp_w8a8_linear_fake_workspace_bytes(m, n, k)
+        ws = torch.empty((wsb,), dtype=torch.uint8, device=x.device)
         _lib.check(lib.mp_w8a8_linear_fake(
             x2.data_ptr(), _DT[x.dtype], m, k, w.data_ptr(), s_ch.data_ptr(), n, _ptr(bias), y.data_ptr(),
             ws.data_ptr(), wsb, _stream()), "mp_w8a8_linear_fake")
