@@ -34,30 +34,6 @@ __device__ __forceinline__ uint4 wide_dq8(uint32_t w0, uint32_t w1, float s) {
   return make_uint4(o[0], o[1], o[2], o[3]);
 }
 
-// Rows [rb, re) and expert of row slot `slot` (dense: the slot-th BM rows; grouped: the slot-th BM-row chunk of
-// an expert, in expert order); false past the last one.
-template <int BM>
-__device__ __forceinline__ bool wide_rows(const mp_dq_args &p, int64_t slot, int64_t &rb, int64_t &re, int &expert) {
-  expert = 0;
-  if (!p.offsets) {
-    rb = slot * BM;
-    re = rb + BM < p.rows ? rb + BM : p.rows;
-    return rb < p.rows;
-  }
-  for (int e = 0; e < p.n_experts; ++e) {
-    const int64_t lo = p.offsets[e], hi = p.offsets[e + 1];
-    const int64_t nch = (hi - lo + BM - 1) / BM;
-    if (slot < nch) {
-      rb = lo + slot * BM;
-      re = rb + BM < hi ? rb + BM : hi;
-      expert = e;
-      return true;
-    }
-    slot -= nch;
-  }
-  return false;
-}
-
 // A workgroup of eight waves (two along M, four along N) makes a tile of up to 256 rows x BN = 128 TN weight rows
 // (SwiGLU: BN / 2 gate rows and the BN / 2 up rows of the same output columns), a wave up to 4 x TN MFMA
 // 32x32x16 tiles: row tiles 2 i + wm, interleaved so that a partly filled tile (the last rows of an expert)
@@ -81,7 +57,7 @@ __device__ __forceinline__ bool wide_rows(const mp_dq_args &p, int64_t slot, int
 template <int DT, int EPI, int TN>
 __global__ __launch_bounds__(512, 2) void dq_wide_kernel(mp_dq_args p, int n_slots, int splits, float *part) {
   constexpr bool SWI = EPI == MP_EPI_SWIGLU;
-  constexpr int TM = 4, WM = 2, WN = 4, BM = 256, BN = 128 * TN;
+  constexpr int TM = 4, WM = 2, WN = 4, BN = 128 * TN;
   constexpr int QB = BN / 8 / 4;  // load instructions per weight stage of a loading wave
   constexpr int BST = BN * 128;
   constexpr int CW = SWI ? 32 : 32 * TN;  // output columns of a wave
@@ -96,7 +72,7 @@ __global__ __launch_bounds__(512, 2) void dq_wide_kernel(mp_dq_args p, int n_slo
   const int64_t col0 = (static_cast<int64_t>(bx / (8 * n_slots)) * 8 + (bx & 7)) * (SWI ? BN / 2 : BN);
   int64_t rb, re;
   int expert;
-  if (col0 >= p.n || !wide_rows<BM>(p, (bx >> 3) % n_slots, rb, re, expert)) return;  // workgroup-uniform
+  if (col0 >= p.n || !wide_rows(p.offsets, p.n_experts, p.rows, (bx >> 3) % n_slots, rb, re, expert)) return;  // workgroup-uniform
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave / WN, wn = wave % WN, half = lane >> 5;
   const uint32_t k = static_cast<uint32_t>(p.k);

@@ -14,28 +14,6 @@ namespace {
 
 constexpr int kI8BK = 128;
 
-// Rows [rb, re) and expert of row slot `slot`; false past the last one.
-__device__ __forceinline__ bool i8w_rows(const mp_i8_args &p, int64_t slot, int64_t &rb, int64_t &re, int &expert) {
-  expert = 0;
-  if (!p.offsets) {
-    rb = slot * 256;
-    re = rb + 256 < p.rows ? rb + 256 : p.rows;
-    return rb < p.rows;
-  }
-  for (int e = 0; e < p.n_experts; ++e) {
-    const int64_t lo = p.offsets[e], hi = p.offsets[e + 1];
-    const int64_t nch = hi > lo ? (hi - lo + 255) / 256 : 0;
-    if (slot < nch) {
-      rb = lo + slot * 256;
-      re = rb + 256 < hi ? rb + 256 : hi;
-      expert = e;
-      return true;
-    }
-    slot -= nch;
-  }
-  return false;
-}
-
 // A workgroup of eight waves (two along M, four along N): up to 256 rows x BN = 128 TN weight rows (SwiGLU: BN / 2
 // gate rows and the BN / 2 matching up rows), a wave up to 4 x TN MFMA 32x32x32 tiles, row tiles 2 i + wm.  LDS:
 // three activation stages of K = 128 sized by the row tiles that are there, weight stages of K = 128 in the rest;
@@ -58,7 +36,7 @@ __global__ __launch_bounds__(512, 2) void i8_wide_kernel(mp_i8_args p, int n_slo
   const int64_t col0 = (static_cast<int64_t>(bx / (8 * n_slots)) * 8 + (bx & 7)) * (SWI ? BN / 2 : BN);
   int64_t rb, re;
   int expert;
-  if (col0 >= p.n || !i8w_rows(p, (bx >> 3) % n_slots, rb, re, expert)) return;  // workgroup-uniform
+  if (col0 >= p.n || !wide_rows(p.offsets, p.n_experts, p.rows, (bx >> 3) % n_slots, rb, re, expert)) return;  // workgroup-uniform
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave / WN, wn = wave % WN, half = lane >> 5;
   const uint32_t k = static_cast<uint32_t>(p.k);

@@ -96,6 +96,9 @@ def test_linear_from_activations_equals_the_two_ops(fake, shape):
 
 @pytest.mark.parametrize("t,e,top,h,inter", [(1, 64, 1, 128, 448), (48, 8, 2, 256, 3136), (700, 8, 2, 3200, 1536),
                                              (300, 2, 1, 12416, 12352), (64, 32, 4, 3072, 896),
+                                             # more experts than a wave has lanes, empty ones between, several chunks
+                                             (100, 65, 1, 256, 128), (40, 200, 2, 128, 192), (1400, 130, 2, 128, 64),
+                                             (2000, 257, 1, 256, 64),
                                              # 64 output columns per workgroup: one group, few tiles, several chunks
                                              (1, 1, 1, 128, 64), (33, 1, 1, 256, 192), (257, 1, 1, 384, 1088), (513, 3, 2, 256, 320)])
 def test_int8_experts_bits(t, e, top, h, inter):
@@ -108,6 +111,8 @@ def test_int8_experts_bits(t, e, top, h, inter):
     s2 = torch.rand(e, h, generator=gen, device="cuda") * 1e-3
     x = torch.randn(t, h, generator=gen, device="cuda").half()
     ids = torch.stack([torch.randperm(e, generator=gen, device="cuda")[:top] for _ in range(t)]).int()
+    if e > 64:  # most of the tokens of the first half go to one expert
+        ids[:t // 2, 0] = torch.where((ids[:t // 2, 1:] == e - 3).any(-1), ids[:t // 2, 0], e - 3)
     routed, rs, _, off = ops.moe_permute_quant(x, ids, e)
     q, s = ops.moe_gmm1_swiglu_quant(routed, rs, w13, s13, off, inter)
     y = ops.moe_gmm2(q, s, w2, s2, off)
