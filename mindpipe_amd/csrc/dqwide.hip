@@ -63,21 +63,18 @@ __global__ __launch_bounds__(512, 2) void dq_wide_kernel(mp_dq_args p, int n_slo
   constexpr int CW = SWI ? 32 : 32 * TN;  // output columns of a wave
   static_assert(!SWI || TN == 2, "gate and up tiles meet in one wave");
   extern __shared__ __attribute__((aligned(16))) int8_t smem_wide[];
-  int bx = static_cast<int>(blockIdx.x), sp = 0;
-  if (TN == 1 && part) {  // the splits of a column tile sit eight apart: on one XCD
-    sp = (bx >> 3) % splits;
-    bx = (bx / (8 * splits)) * 8 + (bx & 7);
-  }
-  // the row slots of a column tile sit eight apart: one XCD, whose L2 then serves their shared weights
-  const int64_t col0 = (static_cast<int64_t>(bx / (8 * n_slots)) * 8 + (bx & 7)) * (SWI ? BN / 2 : BN);
+  const int bx = static_cast<int>(blockIdx.x);
+  constexpr int CPT = SWI ? BN / 2 : BN;  // output columns of a tile
+  int col, slot, sp;
+  if (!wide_tile(bx, static_cast<int>((p.n + CPT - 1) / CPT), n_slots, TN == 1 ? splits : 1, col, slot, sp)) return;
   int64_t rb, re;
   int expert;
-  if (col0 >= p.n || !wide_rows(p.offsets, p.n_experts, p.rows, (bx >> 3) % n_slots, rb, re, expert)) return;  // workgroup-uniform
+  if (!wide_rows(p.offsets, p.n_experts, p.rows, slot, rb, re, expert)) return;  // workgroup-uniform
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave / WN, wn = wave % WN, half = lane >> 5;
   const uint32_t k = static_cast<uint32_t>(p.k);
   const int rows = static_cast<int>(re - rb);
-  const int n_out = static_cast<int>(p.n), c0 = static_cast<int>(col0);
+  const int n_out = static_cast<int>(p.n), c0 = col * CPT;
   const int64_t nb_rows = SWI ? 2 * p.n : p.n;
   const int nt = (rows + 31) / 32;               // row tiles that hold rows
   const int nv = nt > wm ? (nt - wm + 1) / 2 : 0;  // this wave's
@@ -328,11 +325,11 @@ __global__ __launch_bounds__(512, 2) void dq_wide_kernel(mp_dq_args p, int n_slo
 template <int DT, int EPI, int TN>
 int wide_launch(const mp_dq_args &p, int splits, float *part, hipStream_t stream) {
   const int64_t slots = wide_row_slots(p.rows, p.offsets ? p.n_experts : 1);
-  const int64_t cols = mp_cdiv(mp_cdiv(p.n, EPI == MP_EPI_SWIGLU ? 64 * TN : 128 * TN), 8) * 8;
-  if (slots * cols * splits > INT32_MAX) return MP_ERR_SHAPE;
+  const int64_t wgs = mp_cdiv(slots * mp_cdiv(p.n, EPI == MP_EPI_SWIGLU ? 64 * TN : 128 * TN) * splits, 8) * 8;
+  if (wgs > INT32_MAX) return MP_ERR_SHAPE;
   const void *fn = reinterpret_cast<const void *>(dq_wide_kernel<DT, EPI, TN>);
   if (hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, kWLds) != hipSuccess) return MP_ERR_HIP;
-  hipLaunchKernelGGL((dq_wide_kernel<DT, EPI, TN>), dim3(static_cast<unsigned>(slots * cols * splits)), dim3(512), kWLds,
+  hipLaunchKernelGGL((dq_wide_kernel<DT, EPI, TN>), dim3(static_cast<unsigned>(wgs)), dim3(512), kWLds,
                      stream, p, static_cast<int>(slots), splits, part);
   MP_CHECK_LAUNCH();
   return part ? wide_reduce<DT>(part, splits, p.rows, p.n, p.bias, p.y, stream) : MP_OK;

@@ -27,21 +27,18 @@ __global__ __launch_bounds__(512, 2) void i8_wide_kernel(mp_i8_args p, int n_slo
   constexpr int BST = BN * 128;
   static_assert(!(SWI && PART), "forms");
   extern __shared__ __attribute__((aligned(16))) int8_t smem_i8w[];
-  int bx = static_cast<int>(blockIdx.x);
-  int part = 0;
-  if constexpr (PART) {  // the splits of a column tile are eight apart: on one XCD, which then holds its activations
-    part = (bx >> 3) % splits;
-    bx = (bx / (8 * splits)) * 8 + (bx & 7);
-  }
-  const int64_t col0 = (static_cast<int64_t>(bx / (8 * n_slots)) * 8 + (bx & 7)) * (SWI ? BN / 2 : BN);
+  const int bx = static_cast<int>(blockIdx.x);
+  constexpr int CPT = SWI ? BN / 2 : BN;  // output columns of a tile
+  int col, slot, part;
+  if (!wide_tile(bx, static_cast<int>((p.n + CPT - 1) / CPT), n_slots, PART ? splits : 1, col, slot, part)) return;
   int64_t rb, re;
   int expert;
-  if (col0 >= p.n || !wide_rows(p.offsets, p.n_experts, p.rows, (bx >> 3) % n_slots, rb, re, expert)) return;  // workgroup-uniform
+  if (!wide_rows(p.offsets, p.n_experts, p.rows, slot, rb, re, expert)) return;  // workgroup-uniform
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave / WN, wn = wave % WN, half = lane >> 5;
   const uint32_t k = static_cast<uint32_t>(p.k);
   const int rows = static_cast<int>(re - rb);
-  const int n_out = static_cast<int>(p.n), c0 = static_cast<int>(col0);
+  const int n_out = static_cast<int>(p.n), c0 = col * CPT;
   const int64_t nb_rows = SWI ? 2 * p.n : p.n;
   const int nt = (rows + 31) / 32;
   const int nv = nt > wm ? (nt - wm + 1) / 2 : 0;
@@ -405,11 +402,11 @@ __global__ __launch_bounds__(256) void i8_reduce_kernel(const int *__restrict__ 
 template <int EPI, int TN, bool PART>
 int i8w_launch(const mp_i8_args &p, int splits, hipStream_t stream) {
   const int64_t slots = wide_row_slots(p.rows, p.offsets ? p.n_experts : 1);
-  const int64_t cols = mp_cdiv(mp_cdiv(p.n, EPI == MP_EPI_SWIGLU ? 64 * TN : 128 * TN), 8) * 8;
-  if (slots * cols * splits > INT32_MAX) return MP_ERR_SHAPE;
+  const int64_t wgs = mp_cdiv(slots * mp_cdiv(p.n, EPI == MP_EPI_SWIGLU ? 64 * TN : 128 * TN) * splits, 8) * 8;
+  if (wgs > INT32_MAX) return MP_ERR_SHAPE;
   const void *fn = reinterpret_cast<const void *>(i8_wide_kernel<EPI, TN, PART>);
   if (hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, kWLds) != hipSuccess) return MP_ERR_HIP;
-  hipLaunchKernelGGL((i8_wide_kernel<EPI, TN, PART>), dim3(static_cast<unsigned>(slots * cols * splits)), dim3(512), kWLds,
+  hipLaunchKernelGGL((i8_wide_kernel<EPI, TN, PART>), dim3(static_cast<unsigned>(wgs)), dim3(512), kWLds,
                      stream, p, static_cast<int>(slots), splits);
   MP_CHECK_LAUNCH();
   return MP_OK;

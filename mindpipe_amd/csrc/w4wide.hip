@@ -78,20 +78,18 @@ __global__ __launch_bounds__(512, 2) void w4_wide_kernel(mp_w4_wide_args p, int 
   constexpr int CW = SWI ? 32 : 32 * TN;
   static_assert((!SWI || TN == 2) && (!FACT || (TN == 1 && !SWI && DT == MP_F16)), "forms");
   extern __shared__ __attribute__((aligned(16))) int8_t smem_w4[];
-  int bx = static_cast<int>(blockIdx.x), sp = 0;
-  if (TN == 1 && part) {  // the splits of a column tile sit eight apart: on one XCD
-    sp = (bx >> 3) % splits;
-    bx = (bx / (8 * splits)) * 8 + (bx & 7);
-  }
-  const int64_t col0 = (static_cast<int64_t>(bx / (8 * n_slots)) * 8 + (bx & 7)) * (SWI ? BN / 2 : BN);
-  const int64_t rb = static_cast<int64_t>((bx >> 3) % n_slots) * 256;
+  const int bx = static_cast<int>(blockIdx.x);
+  constexpr int CPT = SWI ? BN / 2 : BN;      // output columns of a tile
   const int64_t n_all = SWI ? p.n / 2 : p.n;  // output columns
-  if (col0 >= n_all || rb >= p.m) return;     // workgroup-uniform
+  int col, slot, sp;
+  const bool ok = wide_tile(bx, static_cast<int>((n_all + CPT - 1) / CPT), n_slots, TN == 1 ? splits : 1, col, slot, sp);
+  const int64_t rb = static_cast<int64_t>(slot) * 256;
+  if (!ok || rb >= p.m) return;  // a slot is below p.m / 256; without the test the compiler spills 35 registers of FACT
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave / WN, wn = wave % WN, half = lane >> 5;
   const uint32_t k = static_cast<uint32_t>(p.k);
   const int rows = static_cast<int>(p.m - rb < 256 ? p.m - rb : 256);
-  const int n_out = static_cast<int>(n_all), c0 = static_cast<int>(col0);
+  const int n_out = static_cast<int>(n_all), c0 = col * CPT;
   const int nt = (rows + 31) / 32;
   const int nv = nt > wm ? (nt - wm + 1) / 2 : 0;
   const int ast = nt * 32 * 128, s0 = 3 * ast, b0 = s0 + 2 * SST;
@@ -391,11 +389,11 @@ __global__ __launch_bounds__(512, 2) void w4_wide_kernel(mp_w4_wide_args p, int 
 template <int DT, bool SWI, int TN, bool FACT>
 int w4w_launch(const mp_w4_wide_args &a, int splits, float *part, hipStream_t stream) {
   const int64_t slots = mp_cdiv(a.m, 256);
-  const int64_t cols = mp_cdiv(mp_cdiv(SWI ? a.n / 2 : a.n, SWI ? 64 * TN : 128 * TN), 8) * 8;
-  if (slots * cols * splits > INT32_MAX) return MP_ERR_SHAPE;
+  const int64_t wgs = mp_cdiv(slots * mp_cdiv(SWI ? a.n / 2 : a.n, SWI ? 64 * TN : 128 * TN) * splits, 8) * 8;
+  if (wgs > INT32_MAX) return MP_ERR_SHAPE;
   const void *fn = reinterpret_cast<const void *>(w4_wide_kernel<DT, SWI, TN, FACT>);
   if (hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, kWLds) != hipSuccess) return MP_ERR_HIP;
-  hipLaunchKernelGGL((w4_wide_kernel<DT, SWI, TN, FACT>), dim3(static_cast<unsigned>(slots * cols * splits)), dim3(512),
+  hipLaunchKernelGGL((w4_wide_kernel<DT, SWI, TN, FACT>), dim3(static_cast<unsigned>(wgs)), dim3(512),
                      kWLds, stream, a, static_cast<int>(slots), splits, part);
   MP_CHECK_LAUNCH();
   return part ? wide_reduce<DT>(part, splits, a.m, a.n, a.bias, a.y, stream) : MP_OK;

@@ -28,6 +28,24 @@ __device__ __forceinline__ void wide_phase() {
   __builtin_amdgcn_sched_barrier(0);
 }
 
+// Column tile, row slot and K split of a workgroup, of `cols` x `slots` x `splits`; false if it has none.  Workgroups go to
+// the eight XCDs by turns; the row slots and splits of a column tile stay on one XCD, whose L2 then serves what they
+// share, and column tiles are dealt to the XCDs, but for the last cols % 8: those are cut into eight equal runs.
+// (Dealt as well, they left 20 tiles a third short of work on half of the XCDs and 4 tiles half of the XCDs idle:
+// M = 3072, 5120 x 5120 in int8 126 -> 77 us, M = 12288, N = 1024, K = 4096 106 -> 56 us.)
+__device__ __forceinline__ bool wide_tile(int bx, int cols, int slots, int splits, int &col, int &slot, int &sp) {
+  const int x = bx & 7, per = slots * splits, whole = cols / 8 * per, tail = cols % 8 * per;
+  int j = bx >> 3;
+  const bool dealt = j < whole;
+  j -= dealt ? 0 : whole;
+  const bool ok = dealt || j < tail / 8 + (x < tail % 8 ? 1 : 0);
+  j += dealt ? 0 : x * (tail / 8) + min(x, tail % 8);
+  col = __builtin_amdgcn_readfirstlane(dealt ? j / per * 8 + x : cols / 8 * 8 + j / per);
+  slot = __builtin_amdgcn_readfirstlane(j % per / splits);
+  sp = __builtin_amdgcn_readfirstlane(j % per % splits);
+  return ok;
+}
+
 // Rows [rb, re) and expert of row slot `slot` (dense: the slot-th 256 of `rows`; grouped: the slot-th 256-row chunk of an
 // expert, in expert order); false past the last one.  Called by whole waves; the results are uniform.  Each lane
 // looks at one expert and a prefix sum finds the slot's: taken one after the other, the loads of a search through

@@ -37,6 +37,7 @@ def _rel(a, b):
     (257, 6200, 256, True), (600, 8192, 512, True), (1025, 2568, 1024, False),   # several row slots, one of one row
     (77, 13824, 5120, True), (33, 16392, 8192, False), (200, 4100, 8192, True),  # K split: 2, 1 and 7 ways
     (256, 4096, 4096, True), (1023, 1032, 4352, True), (64, 8200, 9216, True),
+    (2300, 1500, 2048, True), (700, 1540, 4096, False), (3100, 2570, 2048, True),  # 12, 13 and 21 column tiles over the XCDs
     (64, 4096, 512, True), (80, 520, 640, True),                                 # the kernels below the rules
 ])
 def test_w4_linear(dtype, m, n, k, zeros):
@@ -68,6 +69,7 @@ def test_w4_swiglu(dtype, m, n2, k):
     (33, 10300, 256), (64, 10240, 128), (65, 24600, 384), (513, 11010, 256),     # 80 / 96 tiles and up, ragged N
     (1024, 130, 128), (1025, 520, 640), (1300, 4096, 1280),                       # every M from 1024
     (200, 4100, 8192), (40, 4096, 4096), (1000, 1001, 9216), (64, 8192, 28672),   # K split
+    (1100, 40, 256), (5000, 260, 256), (3072, 5120, 256), (700, 1540, 8192),      # 1, 3, 20 and 13 column tiles over the XCDs
     (256, 4096, 4096), (100, 520, 1024),                                          # the kernels below the rules
 ])
 def test_int8_linear_bits(out, m, n, k):
