@@ -424,7 +424,11 @@ int mp_launch_i8_wide(const mp_i8_args &p, int epi, hipStream_t stream) {
   const int64_t cus = mp_cu_count() > 0 ? mp_cu_count() : 256;
   const int64_t groups = p.offsets ? (p.rows < p.n_experts ? p.rows : p.n_experts) : 1;
   const int64_t tiles = mp_cdiv(epi == MP_EPI_SWIGLU ? 2 * p.n : p.n, 256) * groups * mp_cdiv(mp_cdiv(p.rows, groups), 256);
-  const bool two = 4 * tiles >= 3 * cus;  // 256 weight rows per workgroup, see wide_pick (dqwide.hip)
+  // 256 weight rows per workgroup: see wide_pick (dqwide.hip), and for a dense call also where tiles of 128 would be more
+  // than one per CU, a second round of a few: M = 1280, 8192 x 8192 117 -> 103 us, M = 2304, N = 4096, K = 1024 27.7 ->
+  // 22.8 us (23.1 on the large-M kernel); up to 128 rows, bound by the weight stream, 128 (M = 128, N = 40960, K = 8192 95
+  // against 106 us)
+  const bool two = 4 * tiles >= 3 * cus || (!p.offsets && p.rows > 128 && 2 * tiles > cus);
   if (epi == MP_EPI_SWIGLU)
     return two ? i8w_launch<MP_EPI_SWIGLU, 2, false>(p, 1, stream) : i8w_launch<MP_EPI_SWIGLU, 1, false>(p, 1, stream);
   if (epi == MP_EPI_F32) return two ? i8w_launch<MP_EPI_F32, 2, false>(p, 1, stream) : i8w_launch<MP_EPI_F32, 1, false>(p, 1, stream);
