@@ -71,6 +71,10 @@ def test_w4_swiglu(dtype, m, n2, k):
     (200, 4100, 8192), (40, 4096, 4096), (1000, 1001, 9216), (64, 8192, 28672),   # K split
     (1100, 40, 256), (5000, 260, 256), (3072, 5120, 256), (700, 1540, 8192),      # 1, 3, 20 and 13 column tiles over the XCDs
     (256, 4096, 4096), (100, 520, 1024),                                          # the kernels below the rules
+    (48, 4096, 2048), (640, 4096, 8192), (256, 8200, 8192), (256, 16384, 8192),   # no K split: few steps, the mid-M kernel, one slot
+    (128, 33000, 128), (256, 16300, 256), (384, 18400, 256),                      # the tiled kernel's two workgroups per CU
+    (5632, 260, 1024), (6144, 1026, 128), (8192, 4104, 4224), (8448, 4100, 4224), # the large-M kernel
+    (5633, 260, 256), (7936, 4104, 4224),                                         # and next to it
 ])
 def test_int8_linear_bits(out, m, n, k):
     gen = _gen(m, n, k)
