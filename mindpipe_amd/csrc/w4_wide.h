@@ -20,8 +20,7 @@ bool mp_w4_wide_takes(const mp_w4_wide_args &a, bool swiglu);
 // applied to the fp32 sum of a group, as the batched fp16 kernel does (not with swiglu).  partials (fp32
 // [splits, M, N], 16-byte aligned; not with swiglu) or null: K split over workgroups and a second launch.
 int mp_launch_w4_wide(const mp_w4_wide_args &a, bool swiglu, bool rounded, int splits, float *partials, hipStream_t stream);
-int mp_w4_wide_splits(int64_t m, int64_t n, int64_t k);
-// Whether the kernel is the faster one for m rows and n weight rows without a workspace (group 128).
-bool mp_w4_wide_rule(int64_t m, int64_t n, bool swiglu);
+// Whether the kernel is the faster one without a workspace (group 128).
+bool mp_w4_wide_rule(const mp_w4_wide_args &a, bool swiglu);
 // Whether the batched kernel's numerics apply to m rows of an n-column fp16 output (w4a16.hip).
 bool mp_w4_batch_numerics(int64_t m, int64_t n);

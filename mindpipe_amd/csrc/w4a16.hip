@@ -1827,7 +1827,7 @@ static bool mp_batch_takes(int64_t m, int64_t n) {
 
 // Whether the direct-to-LDS kernel (w4wide.hip) runs a group-128 GEMM without a workspace.
 static bool mp_w4_wide(const mp_w4_wide_args &a, bool swiglu) {
-  return mp_w4_wide_rule(a.m, a.n, swiglu) && mp_w4_wide_takes(a, swiglu);
+  return mp_w4_wide_rule(a, swiglu) && mp_w4_wide_takes(a, swiglu);
 }
 
 // Prefill GEMM workgroup: 256 x 128 tiles of 8 waves from M = 256 (measured 8-13% faster than

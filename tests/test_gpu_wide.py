@@ -39,6 +39,9 @@ def _rel(a, b):
     (256, 4096, 4096, True), (1023, 1032, 4352, True), (64, 8200, 9216, True),
     (2300, 1500, 2048, True), (700, 1540, 4096, False), (3100, 2570, 2048, True),  # 12, 13 and 21 column tiles over the XCDs
     (64, 4096, 512, True), (80, 520, 640, True),                                 # the kernels below the rules
+    (300, 6144, 256, True), (128, 12290, 1024, False), (1024, 6150, 768, True),    # the batched and the prefill kernel next to them
+    (128, 16384, 2048, True), (128, 12290, 2048, True), (768, 24580, 1024, False),
+    (48, 11010, 8192, True), (40, 13830, 8192, False),                             # two ways on few CUs, on most
 ])
 def test_w4_linear(dtype, m, n, k, zeros):
     gen = _gen(m, n, k)
@@ -51,7 +54,10 @@ def test_w4_linear(dtype, m, n, k, zeros):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
-@pytest.mark.parametrize("m,n2,k", [(65, 12544, 256), (200, 12304, 512), (300, 6208, 768), (513, 8200, 256), (66, 256, 512)])
+@pytest.mark.parametrize("m,n2,k", [(65, 12544, 256), (200, 12304, 512), (300, 6208, 768), (513, 8200, 256), (66, 256, 512),
+                                    # half of the CUs and more, K from 1024; the kernels before it next to them
+                                    (257, 16640, 1024), (65, 33040, 1024), (700, 11000, 2048), (1025, 6660, 1280), (80, 33040, 768),
+                                    (512, 16384, 1024), (1536, 14336, 1024)])
 def test_w4_swiglu(dtype, m, n2, k):
     """Gate and up in one kernel against the two launches: the same roundings, sums in another order (an output moves by
     a few ulps where gate, up or silu lands on the other side of one)."""
