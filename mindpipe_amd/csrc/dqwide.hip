@@ -66,7 +66,9 @@ __global__ __launch_bounds__(512, 2) void dq_wide_kernel(mp_dq_args p, int n_slo
   const int bx = static_cast<int>(blockIdx.x);
   constexpr int CPT = SWI ? BN / 2 : BN;  // output columns of a tile
   int col, slot, sp;
-  if (!wide_tile(bx, static_cast<int>((p.n + CPT - 1) / CPT), n_slots, TN == 1 ? splits : 1, col, slot, sp)) return;
+  if (!wide_tile(bx, static_cast<int>((p.n + CPT - 1) / CPT), n_slots, TN == 1 ? splits : 1,
+                 wide_by_slot(p.offsets, p.n_experts, n_slots), col, slot, sp))
+    return;
   int64_t rb, re;
   int expert;
   if (!wide_rows(p.offsets, p.n_experts, p.rows, slot, rb, re, expert)) return;  // workgroup-uniform
@@ -325,7 +327,8 @@ __global__ __launch_bounds__(512, 2) void dq_wide_kernel(mp_dq_args p, int n_slo
 template <int DT, int EPI, int TN>
 int wide_launch(const mp_dq_args &p, int splits, float *part, hipStream_t stream) {
   const int64_t slots = wide_row_slots(p.rows, p.offsets ? p.n_experts : 1);
-  const int64_t wgs = mp_cdiv(slots * mp_cdiv(p.n, EPI == MP_EPI_SWIGLU ? 64 * TN : 128 * TN) * splits, 8) * 8;
+  const int64_t wgs = wide_grid(mp_cdiv(p.n, EPI == MP_EPI_SWIGLU ? 64 * TN : 128 * TN), slots, splits,
+                                wide_by_slot(p.offsets, p.n_experts, slots));
   if (wgs > INT32_MAX) return MP_ERR_SHAPE;
   const void *fn = reinterpret_cast<const void *>(dq_wide_kernel<DT, EPI, TN>);
   if (hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, kWLds) != hipSuccess) return MP_ERR_HIP;

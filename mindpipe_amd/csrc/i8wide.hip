@@ -30,7 +30,9 @@ __global__ __launch_bounds__(512, 2) void i8_wide_kernel(mp_i8_args p, int n_slo
   const int bx = static_cast<int>(blockIdx.x);
   constexpr int CPT = SWI ? BN / 2 : BN;  // output columns of a tile
   int col, slot, part;
-  if (!wide_tile(bx, static_cast<int>((p.n + CPT - 1) / CPT), n_slots, PART ? splits : 1, col, slot, part)) return;
+  if (!wide_tile(bx, static_cast<int>((p.n + CPT - 1) / CPT), n_slots, PART ? splits : 1,
+                 wide_by_slot(p.offsets, p.n_experts, n_slots), col, slot, part))
+    return;
   int64_t rb, re;
   int expert;
   if (!wide_rows(p.offsets, p.n_experts, p.rows, slot, rb, re, expert)) return;  // workgroup-uniform
@@ -402,7 +404,8 @@ __global__ __launch_bounds__(256) void i8_reduce_kernel(const int *__restrict__ 
 template <int EPI, int TN, bool PART>
 int i8w_launch(const mp_i8_args &p, int splits, hipStream_t stream) {
   const int64_t slots = wide_row_slots(p.rows, p.offsets ? p.n_experts : 1);
-  const int64_t wgs = mp_cdiv(slots * mp_cdiv(p.n, EPI == MP_EPI_SWIGLU ? 64 * TN : 128 * TN) * splits, 8) * 8;
+  const int64_t wgs = wide_grid(mp_cdiv(p.n, EPI == MP_EPI_SWIGLU ? 64 * TN : 128 * TN), slots, splits,
+                                wide_by_slot(p.offsets, p.n_experts, slots));
   if (wgs > INT32_MAX) return MP_ERR_SHAPE;
   const void *fn = reinterpret_cast<const void *>(i8_wide_kernel<EPI, TN, PART>);
   if (hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, kWLds) != hipSuccess) return MP_ERR_HIP;

@@ -82,7 +82,8 @@ __global__ __launch_bounds__(512, 2) void w4_wide_kernel(mp_w4_wide_args p, int 
   constexpr int CPT = SWI ? BN / 2 : BN;      // output columns of a tile
   const int64_t n_all = SWI ? p.n / 2 : p.n;  // output columns
   int col, slot, sp;
-  const bool ok = wide_tile(bx, static_cast<int>((n_all + CPT - 1) / CPT), n_slots, TN == 1 ? splits : 1, col, slot, sp);
+  const bool ok =
+      wide_tile(bx, static_cast<int>((n_all + CPT - 1) / CPT), n_slots, TN == 1 ? splits : 1, false, col, slot, sp);
   const int64_t rb = static_cast<int64_t>(slot) * 256;
   if (!ok || rb >= p.m) return;  // a slot is below p.m / 256; without the test the compiler spills 35 registers of FACT
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -389,7 +390,7 @@ __global__ __launch_bounds__(512, 2) void w4_wide_kernel(mp_w4_wide_args p, int 
 template <int DT, bool SWI, int TN, bool FACT>
 int w4w_launch(const mp_w4_wide_args &a, int splits, float *part, hipStream_t stream) {
   const int64_t slots = mp_cdiv(a.m, 256);
-  const int64_t wgs = mp_cdiv(slots * mp_cdiv(SWI ? a.n / 2 : a.n, SWI ? 64 * TN : 128 * TN) * splits, 8) * 8;
+  const int64_t wgs = wide_grid(mp_cdiv(SWI ? a.n / 2 : a.n, SWI ? 64 * TN : 128 * TN), slots, splits, false);
   if (wgs > INT32_MAX) return MP_ERR_SHAPE;
   const void *fn = reinterpret_cast<const void *>(w4_wide_kernel<DT, SWI, TN, FACT>);
   if (hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, kWLds) != hipSuccess) return MP_ERR_HIP;

@@ -28,14 +28,30 @@ __device__ __forceinline__ void wide_phase() {
   __builtin_amdgcn_sched_barrier(0);
 }
 
+// Whether wide_tile deals the row slots of the last column tiles (see there).
+__host__ __device__ __forceinline__ bool wide_by_slot(const void *offsets, int n_experts, int64_t slots) {
+  return offsets != nullptr && n_experts > 1 && slots >= 8;
+}
+
 // Column tile, row slot and K split of a workgroup, of `cols` x `slots` x `splits`; false if it has none.  Workgroups go to
 // the eight XCDs by turns; the row slots and splits of a column tile stay on one XCD, whose L2 then serves what they
 // share, and column tiles are dealt to the XCDs, but for the last cols % 8: those are cut into eight equal runs.
 // (Dealt as well, they left 20 tiles a third short of work on half of the XCDs and 4 tiles half of the XCDs idle:
-// M = 3072, 5120 x 5120 in int8 126 -> 77 us, M = 12288, N = 1024, K = 4096 106 -> 56 us.)
-__device__ __forceinline__ bool wide_tile(int bx, int cols, int slots, int splits, int &col, int &slot, int &sp) {
-  const int x = bx & 7, per = slots * splits, whole = cols / 8 * per, tail = cols % 8 * per;
+// M = 3072, 5120 x 5120 in int8 126 -> 77 us, M = 12288, N = 1024, K = 4096 106 -> 56 us.)  With several groups (splits = 1)
+// the last slots of a column are often empty and runs are not equal work: from a slot per XCD, the slots of the last
+// columns are dealt (64 experts, 192 rows each, gate / up of 512 x 2048 with the requantization: 94 ->
+// 61 us).
+__device__ __forceinline__ bool wide_tile(int bx, int cols, int slots, int splits, bool by_slot, int &col, int &slot, int &sp) {
+  const int x = bx & 7, per = slots * splits, whole = cols / 8 * per, last = cols % 8, tail = last * per;
   int j = bx >> 3;
+  if (by_slot && j >= whole) {
+    j -= whole;
+    const int n = last > 0 ? last : 1;
+    slot = __builtin_amdgcn_readfirstlane(j / n * 8 + x);
+    col = __builtin_amdgcn_readfirstlane(cols / 8 * 8 + j % n);
+    sp = 0;
+    return last > 0 && slot < slots;
+  }
   const bool dealt = j < whole;
   j -= dealt ? 0 : whole;
   const bool ok = dealt || j < tail / 8 + (x < tail % 8 ? 1 : 0);
@@ -199,4 +215,10 @@ int wide_reduce(const float *part, int splits, int64_t m, int64_t n, const void 
 // workgroup empty) left half of the engines idle (200 rows, 11008 gate / up pairs x 4096: 74 -> 43 us).
 static inline int64_t wide_row_slots(int64_t rows, int64_t groups) {
   return (rows + 255 * (groups < rows ? groups : rows)) / 256;
+}
+
+// Workgroups of wide_tile's dealing: as many for each XCD as the one with the most has.
+static inline int64_t wide_grid(int64_t cols, int64_t slots, int64_t splits, bool by_slot) {
+  const int64_t tail = by_slot ? mp_cdiv(slots, 8) * (cols % 8) : mp_cdiv(cols % 8 * slots * splits, 8);
+  return 8 * (cols / 8 * slots * splits + tail);
 }
