@@ -2200,7 +2200,10 @@ static bool mp_big_takes(const mp_i8_args &a) {
 //   34 against 32 us) or, up to K = 8192, two per CU and here only 256-column tiles fit once (M = 384, N = 18432, K = 1024
 //   21.5 against 18.0 us; K = 8192 81 against 80 us);
 //   grouped, from three tiles for four CUs, against i8_moe_kernel: the Mixtral-shaped chain at 4 / 16 / 48 / 512 /
-//   1000 tokens 227 / 306 / 309 / 412 / 667 against 283 / 337 / 344 / 457 / 744 us;
+//   1000 tokens 227 / 306 / 309 / 412 / 667 against 283 / 337 / 344 / 457 / 744 us.  Not the down projection of K < 2048, where
+//   a workgroup's start and end weigh most, in two rounds of tiles and more of 32 to 224 rows per expert (64 / 128 experts, 64
+//   rows, 2048 x 768 38 / 76 against 32 / 66 us: i8_moe_kernel works on while it loads the next tile) and from 448 rows
+//   where the 128 x 128 tiles are up to four per CU (8 experts, 512 rows, 2048 x 512 22 against 16 us);
 //   SwiGLU at every size (64 output columns per workgroup where 128 would not fill the CUs): the dense MLP chain
 //   (4096, I = 11008) at 2 / 16 / 96 / 200 / 256 / 400 rows 52 / 53 / 72 / 86 / 91 / 132 against 61 / 62 / 78 / 88 / 94 /
 //   175 us, at 1024 / 4096 rows 236 / 674 against 307 / 1079 us, the expert chain of eight experts (2048, I = 1408) at 8 / 64 /
@@ -2212,6 +2215,11 @@ static bool mp_wide_takes(const mp_i8_args &a, int epilogue) {
   if (a.offsets) {
     const int64_t groups = a.rows < a.n_experts ? a.rows : a.n_experts;
     const int64_t chunks = groups * mp_cdiv(mp_cdiv(a.rows, groups), 256);
+    if (epilogue == MP_EPI_F32 && a.k < 2048 && groups > 1) {
+      const int64_t r = a.rows / groups;
+      if (r >= 32 && r <= 224 && mp_cdiv(a.n, 256) * groups >= 2 * cus) return false;
+      if (r >= 448 && mp_cdiv(a.n, 128) * groups * mp_cdiv(r, 128) <= 4 * cus) return false;
+    }
     return 4 * mp_cdiv(a.n, 128) * chunks >= 3 * cus;
   }
   if (epilogue != MP_EPI_DENSE || a.rows <= 32) return false;
