@@ -91,6 +91,24 @@ def test_experts_equal_the_separate_steps(dtype, t, e, top, h, inter):
     assert _rel(y, ref.double()) <= (2e-3 if dtype == torch.float16 else 8e-3)
 
 
+@pytest.mark.parametrize("t,e,top,inter,one_call", [(1024, 2, 1, 512, False), (384, 2, 1, 512, False), (382, 2, 1, 512, True),
+                                                    (2048, 8, 2, 512, False), (64, 4, 2, 512, True), (1024, 4, 1, 2176, True)])
+def test_experts_route(monkeypatch, t, e, top, inter, one_call):
+    """Few gate / up workgroups on full chunks of rows: the four entry points; else the one call.  The same values."""
+    gen = torch.Generator(device="cuda").manual_seed(t + e)
+    w13, s13, _ = _weight((e, 2 * inter, 256), torch.float16, gen)
+    w2, s2, _ = _weight((e, 256, inter), torch.float16, gen)
+    x = torch.randn(t, 256, generator=gen, device="cuda").half()
+    ids = torch.stack([torch.randperm(e, generator=gen, device="cuda")[:top] for _ in range(t)]).to(torch.int32)
+    tw = torch.rand(t, top, generator=gen, device="cuda")
+    calls, inner = [], ops._moe_fake
+    monkeypatch.setattr(ops, "_moe_fake", lambda *a: calls.append(1) or inner(*a))
+    y = ops.moe_w8a8_forward(x, ids, tw, w13, s13, w2, s2, None, "fake")
+    assert bool(calls) == one_call
+    monkeypatch.setattr(ops, "_moe_fake_takes", lambda *a: not one_call)
+    assert _rel(ops.moe_w8a8_forward(x, ids, tw, w13, s13, w2, s2, None, "fake"), y.double()) <= 2e-3
+
+
 def test_linear_op_traces():
     gen = torch.Generator(device="cuda").manual_seed(3)
     q, s, _ = _weight((72, 128), torch.bfloat16, gen)
