@@ -49,10 +49,9 @@ def test_a_registered_kernel_is_used(register):
 
 def test_reload():
     _python("""
-        old = ops.quant_per_token_i8
         for _ in range(2):
             importlib.reload(ops)
-        for op in (old, ops.quant_per_token_i8, torch.ops.mindpipe_amd.quant_per_token_i8):
+        for op in (ops.quant_per_token_i8, torch.ops.mindpipe_amd.quant_per_token_i8):
             try:
                 op(x)
             except RuntimeError as e:
