@@ -33,7 +33,7 @@ __device__ __forceinline__ uint4 w4w_dq8(uint32_t w, const W4Scale &c) {
       wide_pack2<DT>(fmaf(static_cast<float>(e1[1]), c.s, c.ne), fmaf(static_cast<float>(o1[1]), c.s16, c.no)));
 }
 
-// Eight nibbles as u - z in fp16 (one rounding, none for integer zeros), column order.
+// Eight nibbles as u - z in fp16, column order; exact for a whole z up to 1024.
 __device__ __forceinline__ uint4 w4w_sub8(uint32_t w, whf2_t z) {
   const uint32_t lo = w & 0xFFFFu, hi = w >> 16;
   const uint32_t a = (lo << 12) | lo, b = (hi << 12) | hi;  // nibbles 0 1 | 2 3 of each half at bits 0 and 16, 8 and 24 - 4
@@ -45,6 +45,9 @@ __device__ __forceinline__ uint4 w4w_sub8(uint32_t w, whf2_t z) {
                                          whf2_t{1024, 1024}) - z);
   return make_uint4(o[0], o[1], o[2], o[3]);
 }
+
+// The whole part of a zero point; the rest is exact in fp16.
+__device__ __forceinline__ float w4w_whole(float z) { return fminf(fmaxf(rintf(z), -1024.f), 1024.f); }
 
 template <int DT>
 __device__ __forceinline__ float w4w_f32(uint32_t pair, int hi) {
@@ -194,6 +197,7 @@ __global__ __launch_bounds__(512, 2) void w4_wide_kernel(mp_w4_wide_args p, int 
     i4_t braw[TN];
     W4Scale cs[TN];
     f16_t grp[FACT ? (NV > 0 ? NV : 1) : 1];
+    uint64_t rests = 0;  // FACT: lanes whose column has a zero point that is not whole
     // one K step of 64, P = kt % 4 (two steps to a group and a weight stage, four to a scale stage)
     auto step = [&](auto p_, int kt) {
       constexpr int P = decltype(p_)::value;
@@ -245,8 +249,10 @@ __global__ __launch_bounds__(512, 2) void w4_wide_kernel(mp_w4_wide_args p, int 
 #pragma unroll
             for (int j = 0; j < TN; ++j) {
               const float s = w4w_f32<DT>(sp[j], P >> 1), z = p.zeros ? w4w_f32<DT>(zp[j], P >> 1) : 8.0f;
-              if constexpr (FACT) cs[j] = W4Scale{s, 0.f, 0.f, z};
-              else cs[j] = W4Scale{s, s * 0.0625f, -(1024.f + z) * s, -(64.f + z) * s};
+              if constexpr (FACT) {
+                cs[j] = W4Scale{s, 0.f, 0.f, w4w_whole(z)};
+                rests |= __ballot(cs[j].no != z);
+              } else cs[j] = W4Scale{s, s * 0.0625f, -(1024.f + z) * s, -(64.f + z) * s};
             }
           }
 #pragma unroll
@@ -319,6 +325,32 @@ __global__ __launch_bounds__(512, 2) void w4_wide_kernel(mp_w4_wide_args p, int 
       for (int i = 0; i < NV; ++i)
 #pragma unroll
         for (int r = 0; r < 16; ++r) acc[i][0][r] = fmaf(grp[i][r], cs[0].s, acc[i][0][r]);
+    }
+    if constexpr (FACT && NV > 0) {
+      // The loop took off whole zero points; what is left of them, which fp16 holds, is an operand of its own against
+      // the activations, read again from memory.  (As a branch in the phases it cost 7% where no zero point has a
+      // rest, or the registers: 208 spilled.)
+      if (rests) {
+        const int64_t cz = static_cast<int64_t>(min(colj[0], n_out - 1)) * ng + 2 * first;
+#pragma unroll 1
+        for (int g = 0; g < 2 * nks; ++g) {
+          const float z = mp_h2f(p.zeros[cz + g]), s = mp_h2f(p.scales[cz + g]);
+          const _Float16 d = static_cast<_Float16>(w4w_whole(z) - z);
+          if (!__any(d != static_cast<_Float16>(0))) continue;
+          const uint32_t dd = __builtin_bit_cast(uint32_t, whf2_t{d, d}), at = static_cast<uint32_t>(2 * first + g) * 256;
+#pragma unroll
+          for (int i = 0; i < NV; ++i) {
+            const int r = (i * 2 + wm) * 32 + (lane & 31);
+            const uint32_t vo = r < rows ? static_cast<uint32_t>(r) * k * 2 + 16 * half : kWOob;
+            f16_t t = {};
+#pragma unroll 1
+            for (uint32_t c = 0; c < 256; c += 32)
+              t = wide_mfma<DT>(__builtin_bit_cast(i4_t, mp_buf_load16(arsrc, vo, at + c)), make_uint4(dd, dd, dd, dd), t);
+#pragma unroll
+            for (int q = 0; q < 16; ++q) acc[i][0][q] = fmaf(t[q], s, acc[i][0][q]);
+          }
+        }
+      }
     }
     if constexpr (WMC == 0) wide_phase();
   };

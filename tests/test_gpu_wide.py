@@ -53,6 +53,29 @@ def test_w4_linear(dtype, m, n, k, zeros):
     assert _rel(ops.w4a16_gemm(x, packed, s, z, 128, b), ref + b.double()) <= TOL[dtype]
 
 
+@pytest.mark.parametrize("m,n,k", [(96, 12290, 2048), (40, 13830, 8192), (65, 4100, 16384), (200, 4100, 8192), (289, 4096, 4096),
+                                   (512, 4096, 4096), (77, 13824, 5120)])
+def test_w4_fractional_zero_points(m, n, k):
+    """fp16 rows whose numerics round no weight, with zero points of 4 + 2^-8 in some groups: u - z of 9 to 11 lies between
+    two fp16 values, and rounded it would move every product of the row the same way.  The bias takes the sum off, so
+    that the output shows the fp32 sums: a few roundings per group of their magnitude, and its own."""
+    gen = _gen(m, n, k)
+    u = torch.randint(12, 16, (n, k), generator=gen, device="cuda", dtype=torch.int32)
+    packed = torch.zeros(n, k // 8, device="cuda", dtype=torch.int32)
+    for i in range(8):
+        packed |= u[:, i::8] << (4 * i)
+    s = torch.full((n, k // 128), 2.0 ** -11, device="cuda").half()
+    frac = torch.rand(n, k // 128, generator=gen, device="cuda") < 0.5
+    frac[: n // 2, ::2] = False
+    z = (4.0 + frac * 2.0 ** -8).half()
+    x = torch.randint(1, 4, (1, k), generator=gen, device="cuda").half().expand(m, k).contiguous()
+    ref = (x[:1].double() @ ((u.double() - z.double().repeat_interleave(128, 1)) * 2.0 ** -11).T)[0]
+    b = -ref.half()
+    y = ops.w4a16_gemm(x, packed, s, z, 128, b).double()
+    err, left = (y - (ref + b.double())).abs(), (ref + b.double()).abs()
+    assert bool((err <= 64 * 2.0 ** -24 * ref + 2.0 ** -11 * left).all()), float((err / ref).max())
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("m,n2,k", [(65, 12544, 256), (200, 12304, 512), (300, 6208, 768), (513, 8200, 256), (66, 256, 512),
                                     # half of the CUs and more, K from 1024; the kernels before it next to them
