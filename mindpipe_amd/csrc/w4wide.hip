@@ -505,10 +505,12 @@ extern "C" int mp_w4a16_gemm_ws(const void *x, int64_t m, int64_t k, const int32
   const mp_w4_wide_args a{static_cast<const uint16_t *>(x), reinterpret_cast<const uint32_t *>(w_packed),
                           static_cast<const uint16_t *>(scales), static_cast<const uint16_t *>(zeros),
                           static_cast<const uint16_t *>(bias), static_cast<uint16_t *>(y), x_dtype, m, n, k};
-  // fp16 up to 48 rows, two ways on less than three quarters of the CUs: the batched kernel (M = 40, N = 11008, K = 11008 52.5
-  // against 47.1 us, K = 28672 level; in bf16 the split, 47 against 50 us)
+  // fp16, two ways, up to 48 rows on less than three quarters of the CUs or up to 64 at K <= 4096: the batched kernel (M = 40, N
+  // = 11008, K = 11008 52.5 against 47.1 us, K = 28672 level, in bf16 the split, 47 against 50 us; M = 64, N = 16384, K = 4096 27
+  // against 23.5 us, in bf16 the split, 25.6 against 32 us)
   const int64_t cus = mp_cu_count() > 0 ? mp_cu_count() : 256;
-  const bool few = x_dtype == MP_F16 && m <= 48 && need > 0 && wide_splits(m, n, k) == 2 && 8 * mp_cdiv(n, 128) < 3 * cus;
+  const bool few = x_dtype == MP_F16 && need > 0 && wide_splits(m, n, k) == 2 &&
+                   ((m <= 48 && 8 * mp_cdiv(n, 128) < 3 * cus) || (m <= 64 && k <= 4096));
   if (need == 0 || few || !workspace || workspace_bytes < need || !mp_aligned(workspace, 16) || !x || !w_packed || !scales ||
       !y || (x_dtype != MP_F16 && x_dtype != MP_BF16) || !mp_w4_wide_takes(a, false))
     return mp_w4a16_gemm(x, m, k, w_packed, n, scales, zeros, group_size, bias, y, x_dtype, stream);
