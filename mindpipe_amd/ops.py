@@ -62,17 +62,22 @@ def _dev(t: torch.Tensor):
 # ---------------------------------------------------------------- registration
 globals().pop("_LIGHT", None)  # of an earlier import: a reload defines the operators again
 _LIGHT = torch.library.Library("mindpipe_amd_light", "DEF")
-_PLAIN = (torch.Tensor, torch.nn.Parameter)
+_Tensor, _Parameter = _PLAIN = torch.Tensor, torch.nn.Parameter
+_CONSTANTS = frozenset((type(None), bool, int, float, str, torch.dtype))
 _IMPLS = torch.library._impls  # "ns/op/key" of every torch.library.impl
+# what every eager call looks at, as names of this module (an attribute chain costs as much as the call itself)
+_is_compiling, _is_grad_enabled, _forward_ad = torch.compiler.is_compiling, torch.is_grad_enabled, torch.autograd.forward_ad
+_functorch_level, _tracing_state = torch._C._functorch.peek_interpreter_stack, torch._C._get_tracing_state
+_dispatch_modes, _function_modes = torch._C._len_torch_dispatch_stack, torch._C._len_torch_function_stack
 
 
 class _Op(torch.library.CustomOpDef):
     """The custom op ``torch.ops.<ns>.<name>``, whose eager calls go to ``torch.ops.mindpipe_amd_light.<name>``: the same
     function and fake implementation without the custom op's Python autograd layer.  A call goes to the custom op
     itself under compilation, tracing, dispatch and function modes, functorch transforms and forward-mode AD and where
-    an input requires a gradient (it refuses the backward); its layers cost about 11 us a call, half of an eager one-row linear (23 us).  So does
-    every call without a plain CUDA tensor and, once a kernel or autocast rule is registered for it, every call:
-    the light op knows only this package's kernels."""
+    an input requires a gradient (it refuses the backward); its layers cost about 11 us a call, half of an eager
+    one-row linear (23 us).  So does every call with other than plain CUDA tensors and, once a kernel or autocast rule is
+    registered for it, every call: the light op knows only this package's kernels."""
 
     registered = False  # the user's kernel or autocast rule stands in the custom op
 
@@ -90,17 +95,24 @@ class _Op(torch.library.CustomOpDef):
         return fake
 
     def __call__(self, *args, **kwargs):
-        if (self.registered or self.cuda_impl in _IMPLS or torch.compiler.is_compiling()
-                or torch._C._functorch.peek_interpreter_stack() is not None
-                or torch.autograd.forward_ad._current_level >= 0 or torch._C._len_torch_dispatch_stack()
-                or torch._C._len_torch_function_stack() or torch._C._get_tracing_state() is not None):
-            return super().__call__(*args, **kwargs)
-        grad = torch.is_grad_enabled()
-        for a in (*args, *kwargs.values()):
-            for t in (a,) if isinstance(a, torch.Tensor) else a if isinstance(a, (list, tuple)) else ():
-                if type(t) not in _PLAIN or not t.is_cuda or (grad and t.requires_grad):
-                    return super().__call__(*args, **kwargs)
-        return self.light(*args, **kwargs)
+        if not (self.registered or self.cuda_impl in _IMPLS or _is_compiling() or _functorch_level() is not None
+                or _forward_ad._current_level >= 0 or _dispatch_modes() or _function_modes()
+                or _tracing_state() is not None):
+            grad, device = _is_grad_enabled(), False
+            for a in (*args, *kwargs.values()) if kwargs else args:
+                kind = type(a)
+                if kind is _Tensor or kind is _Parameter:
+                    if (grad and a.requires_grad) or not (device or a.is_cuda):
+                        break
+                    device = True  # the first tensor's: the op itself looks at the others
+                elif kind is list:
+                    if not all(type(t) in _PLAIN and not (grad and t.requires_grad) for t in a):
+                        break
+                elif kind not in _CONSTANTS:
+                    break
+            else:
+                return self.light(*args, **kwargs)
+        return super().__call__(*args, **kwargs)
 
 
 def _op(name, ns="mindpipe_amd"):
