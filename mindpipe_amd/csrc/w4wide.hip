@@ -444,7 +444,9 @@ int w4w_pick(const mp_w4_wide_args &a, bool swiglu, int splits, float *part, hip
 }  // namespace
 
 bool mp_w4_wide_takes(const mp_w4_wide_args &a, bool swiglu) {
-  return a.k % 256 == 0 && a.k <= (1 << 20) && a.n * (a.k / 2) < (int64_t(1) << 31) && mp_aligned(a.x, 16) &&
+  // MP_W4_WIDE=0: the kernels before this one, for measurements
+  static const bool on = !(mp_knob("MP_W4_WIDE") && atoi(mp_knob("MP_W4_WIDE")) == 0);
+  return on && a.k % 256 == 0 && a.k <= (1 << 20) && a.n * (a.k / 2) < (int64_t(1) << 31) && mp_aligned(a.x, 16) &&
          mp_aligned(a.w, 16) && mp_aligned(a.scales, 4) && (!a.zeros || mp_aligned(a.zeros, 4)) && a.m > 0 &&
          a.m <= INT32_MAX && a.n <= INT32_MAX && (!swiglu || a.n % 2 == 0);
 }

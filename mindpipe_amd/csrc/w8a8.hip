@@ -2179,6 +2179,12 @@ static int mp_launch_moe(const mp_i8_args &a, hipStream_t stream) {
   return mp_launch_moe_d<EPI, 1>(a, stream);
 }
 
+// MP_W8_WIDE=0 turns the direct-to-LDS kernel and its K split off (for measurements of the kernels before it).
+static bool mp_wide_on() {
+  static const bool v = !(mp_knob("MP_W8_WIDE") && atoi(mp_knob("MP_W8_WIDE")) == 0);
+  return v;
+}
+
 // Dense calls of thousands of rows that the large-M kernel runs faster than the direct-to-LDS one (i8wide.hip), both
 // graph-timed in turn: whole tiles of 256 rows from M = 5632 at K < 2048 (M = 8192, N = 28672, K = 1024 348 against 395 us,
 // M = 16384, N = 4096 90 against 104 us; at 2048 they are level, M = 8000 49 against 44 us), and from M = 8192 to 9215, where a
@@ -2209,7 +2215,7 @@ static bool mp_big_takes(const mp_i8_args &a) {
 //   175 us, at 1024 / 4096 rows 236 / 674 against 307 / 1079 us, the expert chain of eight experts (2048, I = 1408) at 8 / 64 /
 //   512 tokens 46 / 49 / 69 against 51 / 52 / 71.
 static bool mp_wide_takes(const mp_i8_args &a, int epilogue) {
-  if (epilogue == MP_EPI_AMAX || !mp_i8_wide_takes(a, epilogue)) return false;
+  if (!mp_wide_on() || epilogue == MP_EPI_AMAX || !mp_i8_wide_takes(a, epilogue)) return false;
   const int64_t cus = mp_cu_count() > 0 ? mp_cu_count() : 256;
   if (epilogue == MP_EPI_SWIGLU) return true;
   if (a.offsets) {
@@ -2608,7 +2614,7 @@ extern "C" int mp_w8a8_gemm(const int8_t *qx, const float *s_tok, const int8_t *
 //   nor four ways of whole slots in the mid-M kernel's range (M = 256, 8192 x 8192 38 to 42 against 36 us).
 extern "C" size_t mp_w8a8_gemm_workspace_bytes(int64_t m, int64_t n, int64_t k) {
   if (m <= 32 || m >= 1024 || n <= 0 || k <= 0 || k % 128 != 0 || (k < 8192 && m > 64)) return 0;
-  if (m <= 48 && k < 4096 && (n < 8192 || k < 2560)) return 0;
+  if (!mp_wide_on() || (m <= 48 && k < 4096 && (n < 8192 || k < 2560))) return 0;
   const int s = mp_i8_wide_splits(m, n, k);
   if (s < 2) return 0;
   if (m >= 128 && k < (m == 128 ? 9216 : 11008)) {
