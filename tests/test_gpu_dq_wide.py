@@ -33,7 +33,8 @@ def _rel(a, b):
     (1, 40, 512), (16, 4097, 640), (17, 8200, 896), (32, 16500, 512),           # a few rows: column tiles, tails, K ranges
     (32, 264, 448), (33, 264, 512), (64, 136, 64), (65, 130, 576),              # the tiled kernel: odd steps, ragged N
     (160, 520, 1024), (161, 392, 320), (192, 136, 256), (224, 264, 128),        # stages by row tiles
-    (256, 25000, 192), (257, 12300, 128), (1000, 50000, 64),                    # 256-row column tiles, several row slots
+    (256, 25000, 192), (257, 12300, 128), (1000, 50000, 64),                    # ragged N, several row slots
+    (289, 24842, 448), (1089, 10250, 640),                                      # 256 columns per workgroup, part of a slot
 ])
 def test_linear_edges(dtype, m, n, k):
     gen = torch.Generator(device="cuda").manual_seed(m * 7 + n + k)
@@ -67,6 +68,27 @@ def test_values_equal_codes_times_scale(dtype, k):
         ref = (q.float() * s.float().unsqueeze(-1)).to(dtype).double() @ (w.double() * 2.0 ** -10).T
         y = ops.w8a8_linear_fake(x, w, sw, None)
         assert float((y.double() - ref).norm()) <= TOL[dtype] * float(ref.norm())
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("m,n,k", [(17, 8200, 896), (64, 136, 64), (257, 12300, 128), (6, 64, 16392), (5, 64, 100)])
+def test_rows_of_infinities_and_nan(dtype, m, n, k):
+    """A row with an infinity (its scale is infinite) or NaN: what the separate quantization gives; the others as without it."""
+    gen = torch.Generator(device="cuda").manual_seed(m + n + k)
+    w, sw, wd = _weight((n, k), dtype, gen)
+    x = torch.randn(m, k, generator=gen, device="cuda").to(dtype)
+    clean = ops.w8a8_linear_fake(x, w, sw, None)
+    x[1, k - 1], x[m - 1, 3], x[3, 0] = float("inf"), float("nan"), float("-inf")
+    y = ops.w8a8_linear_fake(x, w, sw, None)
+    q, s = ops.quant_per_token_i8(x, True)
+    values = (q.float() * s.float().unsqueeze(-1)).to(dtype)
+    good = torch.ones(m, dtype=torch.bool, device="cuda")
+    good[[1, 3, m - 1]] = False
+    assert torch.equal(y[good], clean[good])
+    for r in (1, 3, m - 1):
+        assert bool(torch.isfinite(y[r]).any()) == bool(torch.isfinite(values[r]).all())
+    ref = values[[1, 3, m - 1]].double() @ wd.T
+    assert torch.equal(torch.isnan(y[[1, 3, m - 1]]), torch.isnan(ref))
 
 
 @pytest.mark.parametrize("dtype", DTYPES)

@@ -39,12 +39,22 @@ def _case(name, seed=0):
 
     if name.startswith("w4a16"):
         m, dt = {"w4a16_m1": (1, torch.float16), "w4a16_m16": (16, torch.float16),
-                 "w4a16_m300": (300, torch.float16), "w4a16_bf16_m1": (1, torch.bfloat16)}[name]
-        n, k = 512, 1024
+                 "w4a16_m300": (300, torch.float16), "w4a16_bf16_m1": (1, torch.bfloat16),
+                 "w4a16_split": (200, torch.float16), "w4a16_bf16_split": (77, torch.bfloat16)}[name]
+        n, k = (4104, 8192) if "split" in name else (512, 1024)
         w = randn(n, k, dt=dt) * 0.05
         pk, sc, zr, _ = ops.w4_quantize_awq(w, 128, True, return_deq=False)
         x = randn(m, k, dt=dt)
         return (lambda: ops.w4a16_gemm(x, pk, sc, zr, 128, None)), [x]
+    if name.startswith("w8a8_linear"):  # from activations
+        m, n, k = {"w8a8_linear": (256, 768, 1024), "w8a8_linear_split": (200, 4104, 8192), "w8a8_linear_fake": (48, 768, 1024),
+                   "w8a8_linear_fake_bf16": (9, 768, 1024), "w8a8_linear_rule_fake": (300, 768, 1024)}[name]
+        dt = torch.bfloat16 if name.endswith("bf16") else torch.float16
+        x = randn(m, k, dt=dt)
+        w, sw = i8(n, k), torch.rand(n, device=DEV, generator=g) * 0.01
+        if name.startswith("w8a8_linear_fake"):
+            return (lambda: ops.w8a8_linear_fake(x, w, sw, None)), [x]
+        return (lambda: ops.w8a8_linear(x, w, sw, None, dt, name.endswith("rule_fake"))), [x]
     if name.startswith("w8a8"):
         m = {"w8a8_m1": 1, "w8a8_m16": 16, "w8a8_m256": 256, "w8a8_m600": 600}[name]
         n, k = 768, 1024
@@ -58,7 +68,7 @@ def _case(name, seed=0):
         x, r = randn(64, 1024), randn(64, 1024)
         nw = (1 + 0.1 * randn(1024, dt=torch.float32)).half()
         return (lambda: ops.add_rms_norm_dynamic_quant(x, r, nw, 1e-6)), [x, r]
-    if name == "moe_chain":
+    if name in ("moe_chain", "moe_chain_fake"):
         t, h, inter, e, topk = 96, 512, 256, 8, 2
         x = randn(t, h)
         ids = torch.stack([torch.randperm(e, device=DEV, generator=g)[:topk] for _ in range(t)]).to(torch.int32)
@@ -67,6 +77,8 @@ def _case(name, seed=0):
         s13 = torch.rand(e, 2 * inter, device=DEV, generator=g) * 1e-3
         w2 = i8(e, h, inter)
         s2 = torch.rand(e, h, device=DEV, generator=g) * 1e-3
+        if name.endswith("fake"):
+            return (lambda: ops.moe_w8a8_forward(x, ids, tw, w13, s13, w2, s2, None, "fake")), [x, ids, tw]
         return (lambda: ops.moe_w8a8_forward(x, ids, tw, w13, s13, w2, s2)), [x, ids, tw]
     if name == "gmm1_swiglu_requant":
         rows, h, inter = 300, 512, 192
@@ -94,7 +106,9 @@ def _refresh(t, g):
 
 
 NAMES = ["w4a16_m1", "w4a16_m16", "w4a16_m300", "w4a16_bf16_m1", "w8a8_m1", "w8a8_m16", "w8a8_m256", "w8a8_m600",
-         "quant_per_token", "add_rms_norm_quant", "moe_chain", "gmm1_swiglu_requant"]
+         "quant_per_token", "add_rms_norm_quant", "moe_chain", "gmm1_swiglu_requant",
+         "w4a16_split", "w4a16_bf16_split", "w8a8_linear", "w8a8_linear_split", "w8a8_linear_fake", "w8a8_linear_fake_bf16",
+         "w8a8_linear_rule_fake", "moe_chain_fake"]
 
 
 @pytest.mark.parametrize("name", NAMES)

@@ -425,11 +425,11 @@ def test_w8_quantize_export_and_fake_rules():
 # ------------------------------------------------------------------ W8A8 GEMM
 W8_CASES = [(1, 11008, 4096), (16, 11008, 4096), (5, 1000, 256), (17, 512, 1024), (64, 384, 512), (65, 256, 512),
             (256, 1000, 1024), (300, 384, 4096), (7, 100, 48), (1100, 300, 256), (2048, 520, 320),
-            # large-M kernel: four register stages over 3 loop trips, two stages (K % 256 != 0)
+            # direct-to-LDS kernel from M = 1024: four and six row slots, K of 6 and 3 stages
             (1024, 640, 768), (1300, 700, 384),
-            # large-M kernel with odd N: the unpaired store path
+            # the same with odd N
             (1024, 333, 256),
-            # large-M kernel: twenty loop trips, partial row and column tiles
+            # the same: 20 stages, partial row and column tiles
             (1100, 600, 2560),
             # row-contiguous GEMV (M <= 2): K past the last 1 KB chunk, M = 2, tiny K, K = 11008
             (2, 300, 1040), (1, 257, 4112), (2, 64, 16), (1, 100, 11008),

@@ -34,14 +34,17 @@ def _rel(a, b):
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("m,n,k,zeros", [
     (65, 12290, 256, True), (96, 12288, 512, False), (130, 12300, 768, True),   # no workspace: 96 tiles and up, ragged N
+    (289, 24842, 1280, True), (1089, 10250, 1024, False),                        # 256 columns per workgroup, part of a slot
     (257, 6200, 256, True), (600, 8192, 512, True), (1025, 2568, 1024, False),   # several row slots, one of one row
-    (77, 13824, 5120, True), (33, 16392, 8192, False), (200, 4100, 8192, True),  # K split: 2, 1 and 7 ways
+    (77, 13824, 5120, True), (33, 16392, 8192, False), (200, 4100, 8192, True),  # K split: 2, none and 7 ways
     (256, 4096, 4096, True), (1023, 1032, 4352, True), (64, 8200, 9216, True),
     (2300, 1500, 2048, True), (700, 1540, 4096, False), (3100, 2570, 2048, True),  # 12, 13 and 21 column tiles over the XCDs
     (64, 4096, 512, True), (80, 520, 640, True),                                 # the kernels below the rules
     (300, 6144, 256, True), (128, 12290, 1024, False), (1024, 6150, 768, True),    # the batched and the prefill kernel next to them
     (128, 16384, 2048, True), (128, 12290, 2048, True), (768, 24580, 1024, False),
     (48, 11010, 8192, True), (40, 13830, 8192, False),                             # two ways on few CUs, on most
+    (16, 65600, 1280, True), (32, 32800, 2304, False), (16, 32776, 256, True),      # the batched kernel's walk from another step
+    (33, 32800, 2304, True),                                                       # three row parts: from the first
 ])
 def test_w4_linear(dtype, m, n, k, zeros):
     gen = _gen(m, n, k)
@@ -96,6 +99,7 @@ def test_w4_swiglu(dtype, m, n2, k):
 @pytest.mark.parametrize("out", [torch.float16, torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("m,n,k", [
     (33, 10300, 256), (64, 10240, 128), (65, 24600, 384), (513, 11010, 256),     # 80 / 96 tiles and up, ragged N
+    (289, 24842, 384), (1089, 10250, 384),                                        # 256 columns per workgroup, part of a slot
     (1024, 130, 128), (1025, 520, 640), (1300, 4096, 1280),                       # every M from 1024
     (200, 4100, 8192), (40, 4096, 4096), (1000, 1001, 9216), (64, 8192, 28672),   # K split
     (1100, 40, 256), (5000, 260, 256), (3072, 5120, 256), (700, 1540, 8192),      # 1, 3, 20 and 13 column tiles over the XCDs
@@ -115,6 +119,70 @@ def test_int8_linear_bits(out, m, n, k):
     ref = ((acc * st[:, None]) * sc[None]) + b.float()
     assert torch.equal(ops.w8a8_gemm(q, st, w, sc, b, out), ref.to(out))
     assert torch.equal(ops.w8a8_gemm(q, st, w, sc, None, out), ((acc * st[:, None]) * sc[None]).to(out))
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("m,n,k", [(96, 12290, 512), (300, 6144, 256), (200, 4100, 8192), (1025, 2568, 1024)])
+def test_w4_infinite_rows(dtype, m, n, k):
+    """Infinities and NaN in some rows stay in them."""
+    gen = _gen(m, n, k)
+    packed, s, z, _ = _w4(n, k, dtype, gen)
+    x = torch.randn(m, k, generator=gen, device="cuda").to(dtype)
+    clean = ops.w4a16_gemm(x, packed, s, z, 128, None)
+    bad = torch.tensor([0, 33, m - 1], device="cuda")
+    x[0, 5], x[33, k - 1], x[m - 1, k // 2] = float("inf"), float("nan"), float("-inf")
+    y = ops.w4a16_gemm(x, packed, s, z, 128, None)
+    good = torch.ones(m, dtype=torch.bool, device="cuda")
+    good[bad] = False
+    assert not bool(torch.isfinite(y[bad]).any()) and bool(torch.isnan(y[33]).all())
+    assert torch.equal(y[good], clean[good])
+
+
+@pytest.mark.parametrize("m,n,k", [(65, 24600, 384), (200, 4100, 8192), (1025, 520, 640)])
+def test_int8_infinite_scales(m, n, k):
+    """A row's and a column's scale of infinity or NaN: the product's own values, in fp32."""
+    gen = _gen(m, n, k)
+    q = torch.randint(-127, 128, (m, k), generator=gen, device="cuda", dtype=torch.int8)
+    w = torch.randint(-127, 128, (n, k), generator=gen, device="cuda", dtype=torch.int8)
+    q[3] = 0  # 0 x inf
+    st, sc = torch.rand(m, generator=gen, device="cuda") * 0.01, torch.rand(n, generator=gen, device="cuda") * 0.01
+    st[3], st[m - 1], sc[n - 1], sc[7] = float("inf"), float("nan"), float("inf"), 3e38
+    ref = ((q.double() @ w.double().T).float() * st[:, None]) * sc[None]
+    for out in (torch.float32, torch.float16):
+        assert torch.equal(ops.w8a8_gemm(q, st, w, sc, None, out).float().nan_to_num(1.5, 2e38, -2e38),
+                           ref.to(out).float().nan_to_num(1.5, 2e38, -2e38))
+
+
+def test_weight_and_workspace_that_the_split_cannot_take():
+    """A weight off its 16 bytes, a workspace off them, too short or missing: the kernels without the split, the same
+    values."""
+    from mindpipe_amd import _lib
+    lib, (m, n, k) = _lib.load(), (64, 8200, 4096)
+    gen = _gen(m, n, k)
+    q = torch.randint(-127, 128, (m, k), generator=gen, device="cuda", dtype=torch.int8)
+    buf = torch.randint(-127, 128, (n * k + 16,), generator=gen, device="cuda", dtype=torch.int8)
+    st, sc = torch.rand(m, generator=gen, device="cuda") * 0.01, torch.rand(n, generator=gen, device="cuda") * 0.01
+    for off in (0, 8, 1):
+        w = buf[off:off + n * k].view(n, k)
+        ref = (((q.double() @ w.double().T).float() * st[:, None]) * sc[None]).half()
+        assert torch.equal(ops.w8a8_gemm(q, st, w, sc, None, torch.float16), ref)
+    w = buf[:n * k].view(n, k)
+    ref = (((q.double() @ w.double().T).float() * st[:, None]) * sc[None]).half()
+    packed, s, z, wd = _w4(n, 2 * k, torch.float16, gen)
+    x = torch.randn(m, 2 * k, generator=gen, device="cuda").half()
+    need8, need4 = lib.mp_w8a8_gemm_workspace_bytes(m, n, k), lib.mp_w4a16_gemm_workspace_bytes(m, n, 2 * k, 128)
+    assert need8 and need4
+    ws = torch.zeros(max(need8, need4) + 16, dtype=torch.uint8, device="cuda")
+    for ptr, less in ((ws.data_ptr() + 4, 0), (ws.data_ptr(), 1), (None, 0)):
+        y = torch.empty(m, n, device="cuda").half()
+        assert lib.mp_w8a8_gemm_ws(q.data_ptr(), st.data_ptr(), w.data_ptr(), sc.data_ptr(), None, 0, y.data_ptr(),
+                                   ops.MP_F16, m, n, k, ptr, need8 - less, ops._stream()) == 0
+        assert torch.equal(y, ref)
+        y4 = torch.empty(m, n, device="cuda").half()
+        assert lib.mp_w4a16_gemm_ws(x.data_ptr(), m, 2 * k, packed.data_ptr(), n, s.data_ptr(), z.data_ptr(), 128, None,
+                                    y4.data_ptr(), ops.MP_F16, ptr, need4 - less, ops._stream()) == 0
+        assert _rel(y4, x.double() @ wd.T) <= TOL[torch.float16]
+    assert not bool(ws.any())  # none of them wrote to it
 
 
 @pytest.mark.parametrize("fake", [False, True])
@@ -163,6 +231,30 @@ def test_int8_experts_bits(t, e, top, h, inter):
         differ += int(((hh / (hh.abs().amax(-1, keepdim=True) / 127)).round().to(torch.int8) != q[a:b]).sum())
         assert torch.equal(((q[a:b].double() @ w2[i].double().T).float() * s[a:b, None]) * s2[i][None], y[a:b])
     assert differ <= 1e-3 * q.numel()
+
+
+def test_weights_of_2_gib():
+    """Weights past the descriptors of the direct-to-LDS kernel: the large-M kernel, and gate / up on the expert kernel."""
+    gen, k, n = _gen(5), 16384, 131096
+    w = torch.randint(-127, 128, (n, k), generator=gen, device="cuda", dtype=torch.int8)
+    sc = torch.rand(n, generator=gen, device="cuda") * 1e-3
+    q = torch.randint(-127, 128, (1100, k), generator=gen, device="cuda", dtype=torch.int8)
+    st = torch.rand(1100, generator=gen, device="cuda") * 0.01
+    cols = torch.cat([torch.arange(8, device="cuda"), torch.arange(n - 16, n, device="cuda"),
+                      torch.randint(0, n, (40,), generator=gen, device="cuda")])
+    y = ops.w8a8_gemm(q, st, w, sc, None, torch.float16)
+    acc = (q.double() @ w[cols].double().T).float()
+    assert torch.equal(y[:, cols], ((acc * st[:, None]) * sc[cols][None]).half())
+    del y
+    rows, inter = 40, n // 2
+    codes, s = ops.moe_gmm1_swiglu_quant(q[:rows], st[:rows].contiguous(), w.unsqueeze(0), sc.unsqueeze(0),
+                                         torch.tensor([0, rows], device="cuda", dtype=torch.int64), inter)
+    gu = torch.cat([(q[:rows].double() @ w[i:i + 8192].double().T).float() for i in range(0, n, 8192)], 1)
+    gu = (gu * st[:rows, None]) * sc
+    hh = gu[:, :inter] / (1 + torch.exp(-gu[:, :inter])) * gu[:, inter:]
+    assert torch.allclose(s.view(-1), hh.abs().amax(-1) / 127, rtol=1e-5)
+    diff = ((hh / s.view(-1, 1)).round().int() - codes.int()).abs()
+    assert int(diff.max()) <= 1 and int((diff != 0).sum()) <= 1e-3 * codes.numel()
 
 
 @pytest.mark.parametrize("rows,inter", [(1, 63), (3, 1027), (2, 2052), (300, 1030), (2049, 260)])
