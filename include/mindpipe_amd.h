@@ -216,7 +216,8 @@ int mp_w8a8_gemm_fake(const int8_t *qx, const float *s_tok, const int8_t *w, con
 
 /* The same linear from the activations themselves, x [M,K] in dtype (fp16 / bf16): their per-token
  * fake-quantized values r(q * s), and at sizes that leave CUs idle the fp32 sums of K splits, go to
- * the workspace (mp_w8a8_linear_fake_workspace_bytes, 16-byte aligned), and y = F.linear(values, r(w * s_ch), bias) in dtype.  Equal to mp_quant_per_token_i8
+ * the workspace (mp_w8a8_linear_fake_workspace_bytes, 16-byte aligned), and
+ * y = F.linear(values, r(w * s_ch), bias) in dtype.  Equal to mp_quant_per_token_i8
  * (MP_SCALE_FAKE) followed by mp_w8a8_gemm_fake up to the order of the fp32 sums. */
 size_t mp_w8a8_linear_fake_workspace_bytes(int64_t m, int64_t n, int64_t k);
 int mp_w8a8_linear_fake(const void *x, int dtype, int64_t m, int64_t k, const int8_t *w, const float *s_ch,
@@ -334,8 +335,8 @@ int mp_moe_unpermute_combine(const float *y, const int32_t *row_of_slot, const f
  * mp_moe_unpermute_combine with MP_SCALE_FAKE in x_dtype (fp16 / bf16), on 16-bit values between
  * the steps.  w13 int8 [E, 2I, H] (gate rows first), w2 int8 [E, H, I], fp32 row scales; topk_ids
  * int32 and topk_w fp32 [T, top_k] (ids outside [0, E) contribute nothing); out [T, H] in
- * out_dtype (fp16 / bf16).  H % 64 == 0, I % 64 == 0, 2 * I * H < 2^31, w13 / w2 / out / workspace 16-byte aligned, top_k <= 64;
- * anything else: MP_ERR_SHAPE / MP_ERR_ALIGN, and the four entry points. */
+ * out_dtype (fp16 / bf16).  H % 64 == 0, I % 64 == 0, 2 * I * H < 2^31, w13 / w2 / workspace 16-byte and out 8-byte
+ * aligned, top_k <= 64; anything else: MP_ERR_SHAPE / MP_ERR_ALIGN, and the four entry points. */
 size_t mp_moe_fake_workspace_bytes(int64_t t, int64_t h, int64_t inter, int top_k, int n_experts);
 int mp_moe_fake_forward(const void *x, int x_dtype, int64_t t, int64_t h, const int32_t *topk_ids,
                         const float *topk_w, int top_k, int n_experts, const int8_t *w13, const float *s13,

@@ -112,12 +112,12 @@ __global__ __launch_bounds__(512, 2) void dq_wide_kernel(mp_dq_args p, int n_slo
   // K steps [first, first + nkt) and their weight stages (a split starts and ends at a weight stage)
   const int all = static_cast<int>(k / kWBK), first = TN == 1 ? all / 2 * sp / splits * 2 : 0;
   const int nkt = (TN == 1 && sp + 1 < splits ? all / 2 * (sp + 1) / splits * 2 : all) - first, nkb = (nkt + 1) / 2;
-  // XCDs and experts start at different places of K and wrap around: in step, every workgroup would ask for the
-  // same 128 bytes of rows that lie K bytes apart, which at K = 4096 is a few of the memory channels at a time
-  // (32 rows, 65536 x 4096, a start of its own for each column tile: 74 -> 59 us).  The workgroups of an XCD
-  // that share activation rows stay in step: the experts' rows together exceed its L2.  An odd number of steps starts at 0: its last weight stage's second half
-  // is the next row's bytes (or, past the buffer, zeros) and never read.  Stages past the end are loaded and
-  // never read.
+  // XCDs and experts start at different places of K and wrap around: in step, every workgroup would ask for the same
+  // 128 bytes of rows that lie K bytes apart, which at K = 4096 is a few of the memory channels at a time (32 rows,
+  // 65536 x 4096, a start of its own for each column tile: 74 -> 59 us).  The workgroups of an XCD that share
+  // activation rows stay in step: the experts' rows together exceed its L2.  An odd number of steps starts at 0: its
+  // last weight stage's second half is the next row's bytes (or, past the buffer, zeros) and never read.  Stages past
+  // the end are loaded and never read.
   const int rot = nkt & 1 ? 0 : ((bx & 7) * nkb / 8 + expert * 5) % nkb;
   auto wrap = [](int t, int n) { return min(t < n ? t : t - n, n - 1); };
   auto load_a = [&](int kt, int slot, int q) {

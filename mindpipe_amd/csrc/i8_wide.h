@@ -1,4 +1,4 @@
-// The direct-to-LDS int8 GEMM (i8wide.hip) for up to a few hundred rows per weight.
+// The direct-to-LDS int8 GEMM (i8wide.hip), dense (from 33 rows to thousands) and grouped by expert.
 #pragma once
 #include "i8_gemm.h"
 

@@ -458,22 +458,24 @@ int mp_launch_w4_wide(const mp_w4_wide_args &a, bool swiglu, bool rounded, int s
   return w4w_launch<MP_F16, false, 1, true>(a, splits, partials, stream);
 }
 
-// SwiGLU (a workgroup makes 128 output columns of up to 256 rows): from more than half of the CUs, where the prefill kernel's
-// workgroups of half the size come to more than one round (M = 768, 2 I = 11264, K = 2048 (132 workgroups) 61 against 88
-// us, M = 300, 2 I = 22016, K = 4096 93 against 144 us, M = 2048 354 against 475 us); below that the kernels before
-// it are faster (M = 65, 2 I = 12288, K = 4096 in bf16 62 against 35 us, M = 256, 2 I = 22016 93 against 78 us, M = 512, 2 I = 16384
-// 94 against 85 us), as at K = 1024 with a second round of up to half the CUs (M = 1536, 2 I = 14336 88 against 82 us).
+// SwiGLU (a workgroup makes 128 output columns of up to 256 rows): from more than half of the CUs, where the prefill
+// kernel's workgroups of half the size come to more than one round (M = 768, 2 I = 11264, K = 2048 (132 workgroups) 61
+// against 88 us, M = 300, 2 I = 22016, K = 4096 93 against 144 us, M = 2048 354 against 475 us); below that the kernels
+// before it are faster (M = 65, 2 I = 12288, K = 4096 in bf16 62 against 35 us, M = 256, 2 I = 22016 93 against 78 us,
+// M = 512, 2 I = 16384 94 against 85 us), as at K = 1024 with a second round of up to half the CUs (M = 1536, 2 I =
+// 14336 88 against 82 us).
 //
-// Linears from 96 tiles of 256 rows x 128 columns.  Against the prefill kernel (M = 2048, N = 12288 230 against 265 us, M = 512, N =
-// 22016 126 against 152 us, M = 600, 8192 x 8192 112 against 153 us, M = 128, N = 28672, K = 8192 93 against 133 us; with 32 tiles
-// 56 against 33 us) from K = 1024: below it a tile's start and end count for more (M = 1024, N = 20480, K = 256 43 against 32
-// us, K = 512 53 against 44 us), at 1024 not in a second round of up to half the CUs (M = 768, N = 24576 74 against 69 us), nor up
-// to 128 rows from three quarters of the CUs' 256-column tiles (M = 128, N = 65536 32.4 against 29.7 us), nor, below 4096, up to
-// 128 rows with a second round of 128-column tiles on less than half of the CUs (M = 128, N = 40960, K = 2048 51 against 45 us).
-// Against the batched kernel's row parts only in fp16, in one row slot and from K = 2048 (M = 128, N = 12288, K = 2048 in fp16 /
-// bf16 19.0 / 22.9 against 20.0 / 20.6 us, K = 1024 15.0 against 12.2 us, M = 128, N = 16384, K = 2048 24 against 20 us, M = 300, N =
-// 6144, K = 2048 31.8 against 21.7 us), and below K = 1024, where those are slow (M = 128, N = 16384, K = 256 8.6 against 11.9 us),
-// but for a second slot of a few rows.
+// Linears from 96 tiles of 256 rows x 128 columns.  Against the prefill kernel (M = 2048, N = 12288 230 against 265 us,
+// M = 512, N = 22016 126 against 152 us, M = 600, 8192 x 8192 112 against 153 us, M = 128, N = 28672, K = 8192 93
+// against 133 us; with 32 tiles 56 against 33 us) from K = 1024: below it a tile's start and end count for more (M =
+// 1024, N = 20480, K = 256 43 against 32 us, K = 512 53 against 44 us), at 1024 not in a second round of up to half the
+// CUs (M = 768, N = 24576 74 against 69 us), nor up to 128 rows from three quarters of the CUs' 256-column tiles (M =
+// 128, N = 65536 32.4 against 29.7 us), nor, below 4096, up to 128 rows with a second round of 128-column tiles on less
+// than half of the CUs (M = 128, N = 40960, K = 2048 51 against 45 us).  Against the batched kernel's row parts only in
+// fp16, in one row slot and from K = 2048 (M = 128, N = 12288, K = 2048 in fp16 / bf16 19.0 / 22.9 against 20.0 / 20.6
+// us, K = 1024 15.0 against 12.2 us, M = 128, N = 16384, K = 2048 24 against 20 us, M = 300, N = 6144, K = 2048 31.8
+// against 21.7 us), and below K = 1024, where those are slow (M = 128, N = 16384, K = 256 8.6 against 11.9 us), but for
+// a second slot of a few rows.
 bool mp_w4_wide_rule(const mp_w4_wide_args &a, bool swiglu) {
   if (a.m <= 64) return false;
   const int64_t cus = mp_cu_count() > 0 ? mp_cu_count() : 256, slots = mp_cdiv(a.m, 256);
@@ -489,10 +491,10 @@ bool mp_w4_wide_rule(const mp_w4_wide_args &a, bool swiglu) {
   return a.k >= 1024 && !short_tail && (a.k >= 2048 || a.m > 128 || 4 * wide < 3 * cus);
 }
 
-// K split from 2^32 multiply-adds, up to 256 rows below K = 4096 above them (less is what the second launch costs): measured
-// against the batched kernel M = 77, N = 13824, K = 5120 36 against 55 us, M = 256, N = 4096, K = 11008 / 4096 41 / 29 against
-// 85 / 33 us, M = 64, N = 8192, K = 28672 76 against 85 us; M = 65, 4096 x 4096 24 against 18 us, M = 256, N = 8192, K = 2048 28
-// against 23 us.
+// K split from 2^32 multiply-adds, up to 256 rows below K = 4096 above them (less is what the second launch costs):
+// measured against the batched kernel M = 77, N = 13824, K = 5120 36 against 55 us, M = 256, N = 4096, K = 11008 / 4096
+// 41 / 29 against 85 / 33 us, M = 64, N = 8192, K = 28672 76 against 85 us; M = 65, 4096 x 4096 24 against 18 us, M =
+// 256, N = 8192, K = 2048 28 against 23 us.
 extern "C" size_t mp_w4a16_gemm_workspace_bytes(int64_t m, int64_t n, int64_t k, int group_size) {
   if (m <= 32 || m >= 1024 || n <= 0 || k <= 0 || group_size != 128 || k % 256 != 0) return 0;
   if (k > (1 << 20) || n > INT32_MAX || m * n < (int64_t(1) << 32) / k + (m <= 256 && k < 4096)) return 0;
@@ -507,9 +509,9 @@ extern "C" int mp_w4a16_gemm_ws(const void *x, int64_t m, int64_t k, const int32
   const mp_w4_wide_args a{static_cast<const uint16_t *>(x), reinterpret_cast<const uint32_t *>(w_packed),
                           static_cast<const uint16_t *>(scales), static_cast<const uint16_t *>(zeros),
                           static_cast<const uint16_t *>(bias), static_cast<uint16_t *>(y), x_dtype, m, n, k};
-  // fp16, two ways, up to 48 rows on less than three quarters of the CUs or up to 64 at K <= 4096: the batched kernel (M = 40, N
-  // = 11008, K = 11008 52.5 against 47.1 us, K = 28672 level, in bf16 the split, 47 against 50 us; M = 64, N = 16384, K = 4096 27
-  // against 23.5 us, in bf16 the split, 25.6 against 32 us)
+  // fp16, two ways, up to 48 rows on less than three quarters of the CUs or up to 64 at K <= 4096: the batched kernel
+  // (M = 40, N = 11008, K = 11008 52.5 against 47.1 us, K = 28672 level, in bf16 the split, 47 against 50 us; M = 64, N
+  // = 16384, K = 4096 27 against 23.5 us, in bf16 the split, 25.6 against 32 us)
   const int64_t cus = mp_cu_count() > 0 ? mp_cu_count() : 256;
   const bool few = x_dtype == MP_F16 && need > 0 && wide_splits(m, n, k) == 2 &&
                    ((m <= 48 && 8 * mp_cdiv(n, 128) < 3 * cus) || (m <= 64 && k <= 4096));

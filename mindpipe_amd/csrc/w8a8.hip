@@ -2186,34 +2186,38 @@ static bool mp_wide_on() {
 }
 
 // Dense calls of thousands of rows that the large-M kernel runs faster than the direct-to-LDS one (i8wide.hip), both
-// graph-timed in turn: whole tiles of 256 rows from M = 5632 at K < 2048 (M = 8192, N = 28672, K = 1024 348 against 395 us,
-// M = 16384, N = 4096 90 against 104 us; at 2048 they are level, M = 8000 49 against 44 us), and from M = 8192 to 9215, where a
-// column tile's row slots are one round of an XCD and no two column tiles share activations (N = 4096, K = 11008 338
-// against 366 us, N = 13824, K = 5120 568 against 621 us; 4096 x 4096 138 against 129 us, M = 6144 and 10240 the other way).
+// graph-timed in turn: whole tiles of 256 rows from M = 5632 at K < 2048 (M = 8192, N = 28672, K = 1024 348 against 395
+// us, M = 16384, N = 4096 90 against 104 us; at 2048 they are level, M = 8000 49 against 44 us), and from M = 8192 to
+// 9215, where a column tile's row slots are one round of an XCD and no two column tiles share activations (N = 4096, K
+// = 11008 338 against 366 us, N = 13824, K = 5120 568 against 621 us; 4096 x 4096 138 against 129 us, M = 6144 and
+// 10240 the other way).
 static bool mp_big_takes(const mp_i8_args &a) {
   if (a.rows < 5632 || a.rows % 256 != 0 || a.k % (2 * kBigBK) != 0) return false;
   return a.k < 2048 || (a.rows >= 8192 && a.rows < 9216 && a.n * a.k > (int64_t(1) << 24) && a.k < 16384);
 }
 
 // Whether the direct-to-LDS kernel (i8wide.hip) is the faster one.  Graph-timed calls, all in turn:
-//   dense, M >= 1024, against the large-M kernel (see mp_big_takes): M = 2048, 4096 x 4096 56 against 77 us, M = 2000, N = 4096,
-//   K = 11008 128 against 192 us, M = 1500, 8192 x 8192 130 against 156 us, M = 4096, N = 11008 180 against 202 us;
+//   dense, M >= 1024, against the large-M kernel (see mp_big_takes): M = 2048, 4096 x 4096 56 against 77 us, M = 2000,
+//   N = 4096, K = 11008 128 against 192 us, M = 1500, 8192 x 8192 130 against 156 us, M = 4096, N = 11008 180 against
+//   202 us;
 //   dense, 33 <= M < 1024, from 96 tiles of 256 rows x 128 columns (80 up to 64 rows) where the mid-M kernel does not
-//   run: M = 800, 8192 x 8192 86 against 109 us, M = 512, N = 11008 46 against 54 us, M = 64, N = 11008 / 28672 26.5 / 35
-//   against 31 / 44 us (the mid-M kernel's smaller tiles win at M = 256, N = 11008: 29 against 39 us).  Not, against the
-//   tiled kernel's two workgroups of 128 x 128 per CU, up to 128 rows and below K = 5120 with less than half a round of tiles
-//   more than the CUs (M = 128, N = 40960, K = 2048 37 against 30 us; N = 49152 28 against 31 us), above them where its tiles fit one per CU (M = 256, N = 16384, K = 4096
-//   34 against 32 us) or, up to K = 8192, two per CU and here only 256-column tiles fit once (M = 384, N = 18432, K = 1024
-//   21.5 against 18.0 us; K = 8192 81 against 80 us);
-//   grouped, from three tiles for four CUs, against i8_moe_kernel: the Mixtral-shaped chain at 4 / 16 / 48 / 512 /
-//   1000 tokens 227 / 306 / 309 / 412 / 667 against 283 / 337 / 344 / 457 / 744 us.  Not the down projection of K < 2048, where
-//   a workgroup's start and end weigh most, in two rounds of tiles and more of 32 to 224 rows per expert (64 / 128 experts, 64
-//   rows, 2048 x 768 38 / 76 against 32 / 66 us: i8_moe_kernel works on while it loads the next tile) and from 448 rows
-//   where the 128 x 128 tiles are up to four per CU (8 experts, 512 rows, 2048 x 512 22 against 16 us);
-//   SwiGLU at every size (64 output columns per workgroup where 128 would not fill the CUs): the dense MLP chain
-//   (4096, I = 11008) at 2 / 16 / 96 / 200 / 256 / 400 rows 52 / 53 / 72 / 86 / 91 / 132 against 61 / 62 / 78 / 88 / 94 /
-//   175 us, at 1024 / 4096 rows 236 / 674 against 307 / 1079 us, the expert chain of eight experts (2048, I = 1408) at 8 / 64 /
-//   512 tokens 46 / 49 / 69 against 51 / 52 / 71.
+//   run: M = 800, 8192 x 8192 86 against 109 us, M = 512, N = 11008 46 against 54 us, M = 64, N = 11008 / 28672 26.5 /
+//   35 against 31 / 44 us (the mid-M kernel's smaller tiles win at M = 256, N = 11008: 29 against 39 us).  Not, against
+//   the tiled kernel's two workgroups of 128 x 128 per CU, up to 128 rows and below K = 5120 with less than half a
+//   round of tiles more than the CUs (M = 128, N = 40960, K = 2048 37 against 30 us; N = 49152 28 against 31 us), above
+//   them where its tiles fit one per CU (M = 256, N = 16384, K = 4096 34 against 32 us) or, up to K = 8192, two per CU
+//   and here only 256-column tiles fit once (M = 384, N = 18432, K = 1024 21.5 against 18.0 us; K = 8192 81 against 80
+//   us);
+//   grouped, from three tiles for four CUs, against i8_moe_kernel: the Mixtral-shaped chain at 4 / 16 / 48 / 512 / 1000
+//   tokens 227 / 306 / 309 / 412 / 667 against 283 / 337 / 344 / 457 / 744 us.  Not the down projection of K < 2048,
+//   where a workgroup's start and end weigh most, in two rounds of tiles and more of 32 to 224 rows per expert (64 /
+//   128 experts, 64 rows, 2048 x 768 38 / 76 against 32 / 66 us: i8_moe_kernel works on while it loads the next tile)
+//   and from 448 rows where the 128 x 128 tiles are up to four per CU (8 experts, 512 rows, 2048 x 512 22 against 16
+//   us);
+//   SwiGLU at every size (64 output columns per workgroup where 128 would not fill the CUs): the dense MLP chain (4096,
+//   I = 11008) at 2 / 16 / 96 / 200 / 256 / 400 rows 52 / 53 / 72 / 86 / 91 / 132 against 61 / 62 / 78 / 88 / 94 / 175
+//   us, at 1024 / 4096 rows 236 / 674 against 307 / 1079 us, the expert chain of eight experts (2048, I = 1408) at 8 /
+//   64 / 512 tokens 46 / 49 / 69 against 51 / 52 / 71.
 static bool mp_wide_takes(const mp_i8_args &a, int epilogue) {
   if (!mp_wide_on() || epilogue == MP_EPI_AMAX || !mp_i8_wide_takes(a, epilogue)) return false;
   const int64_t cus = mp_cu_count() > 0 ? mp_cu_count() : 256;
@@ -2603,14 +2607,15 @@ extern "C" int mp_w8a8_gemm(const int8_t *qx, const float *s_tok, const int8_t *
   return mp_launch_i8_gemm(a, MP_EPI_DENSE, reinterpret_cast<hipStream_t>(stream));
 }
 
-// K split where K is long or the rows few: measured (graph-timed calls with the row quant) against the kernels
-// without it M = 200, N = 4096, K = 11008 38 against 56 us, M = 100, 8192 x 8192 36 against 47 us, M = 64, N = 8192, K = 28672
+// K split where K is long or the rows few: measured (graph-timed calls with the row quant) against the kernels without
+// it M = 200, N = 4096, K = 11008 38 against 56 us, M = 100, 8192 x 8192 36 against 47 us, M = 64, N = 8192, K = 28672
 // 74 against 163 us, M = 40, 4096 x 4096 18 against 21 us; M = 256, 4096 x 4096 26 against 23 us.  Not
-//   up to 48 rows below K = 4096 (M = 48, N = 4096, K = 2048 12.1 against 9.8 us, M = 33, K = 3584 13.4 against 11.6 us), but for
-//   8192 columns (M = 48, K = 3072 15.4 against 19.7 us);
-//   below K = 11008 (9216 at 128 rows) two or three ways where the mid-M kernel runs or the rows are one slot (M = 640, N =
-//   4096, K = 8192 41 against 34.5 us, M = 512, N = 5120, K = 9216 43.7 against 40.2 us, M = 256, N = 16384, K = 8192 58 against
-//   54 us), but three ways for a last slot of a few rows (M = 320, N = 5120, K = 8192 32 against 36 us);
+//   up to 48 rows below K = 4096 (M = 48, N = 4096, K = 2048 12.1 against 9.8 us, M = 33, K = 3584 13.4 against 11.6
+//   us), but for 8192 columns (M = 48, K = 3072 15.4 against 19.7 us);
+//   below K = 11008 (9216 at 128 rows) two or three ways where the mid-M kernel runs or the rows are one slot (M = 640,
+//   N = 4096, K = 8192 41 against 34.5 us, M = 512, N = 5120, K = 9216 43.7 against 40.2 us, M = 256, N = 16384, K =
+//   8192 58 against 54 us), but three ways for a last slot of a few rows (M = 320, N = 5120, K = 8192 32 against 36
+//   us);
 //   nor four ways of whole slots in the mid-M kernel's range (M = 256, 8192 x 8192 38 to 42 against 36 us).
 extern "C" size_t mp_w8a8_gemm_workspace_bytes(int64_t m, int64_t n, int64_t k) {
   if (m <= 32 || m >= 1024 || n <= 0 || k <= 0 || k % 128 != 0 || (k < 8192 && m > 64)) return 0;
