@@ -225,8 +225,12 @@ class SmoothQuantLinear(nn.Module):
         bias = None if self.bias is None else self.bias.to(torch.bfloat16)
         return ops.w8a8_linear_fake(x.contiguous(), self.weight, self.weight_scale, bias)
 
-    def _linear(self, x, q, s):
-        """The linear's output on the input's codes, before any output quant (not the bf16 fake-rule linear's)."""
+    def _linear(self, x, fake, q, s):
+        """The linear's output on the input's codes, before any output quant (in bf16 by the fake rule the chain step by step;
+        the module's own calls take the values: ``_linear_values``)."""
+        if fake and x.dtype == torch.bfloat16:
+            bias = None if self.bias is None else self.bias.to(torch.bfloat16)
+            return ops.w8a8_gemm_fake(q, s.float().contiguous(), self.weight, self.weight_scale, bias, x.dtype)
         return ops.w8a8_gemm(q, s.float().contiguous(), self.weight, self.weight_scale, self.bias, x.dtype)
 
     def _fused_output_quant(self, x, fake: bool) -> bool:
@@ -259,7 +263,7 @@ class SmoothQuantLinear(nn.Module):
         fake, q, s = self._input_codes(x)
         if self._fused_output_quant(x, fake):
             return self._output_codes(q, s, x.dtype)
-        return ops.quant_per_token_i8(self._linear(x, q, s).contiguous(), True)
+        return ops.quant_per_token_i8(self._linear(x, fake, q, s).contiguous(), True)
 
     @staticmethod
     def from_float(module, weight_bits=8, activation_bits=8, act_quant="per_token", quantize_output=False,
