@@ -519,9 +519,9 @@ def test_w8a8_gemm_large_rows_subset():
 
 @pytest.mark.parametrize("out", ["fp16", "bf16"])
 def test_w8a8_gemm_persistent_partial_tiles(out):
-    """M = 4100, N = 5000, K = 512: 17 x 20 tiles of 256 x 256 over a persistent grid (more tiles than
-    CUs), with a partial last row tile (4 rows) and column tile (136 columns); bit-exact on sampled
-    rows (those of the partial tile included) x all columns."""
+    """M = 4100, N = 5000, K = 512: 17 x 20 tiles of 256 x 256 on the direct-to-LDS kernel (more tiles than
+    CUs; the persistent large-M kernel takes other sizes), with a partial last row tile (4 rows) and column
+    tile (136 columns); bit-exact on sampled rows (those of the partial tile included) x all columns."""
     _say("w8a8 persistent partial tiles", out)
     m, n, k = 4100, 5000, 512
     gen = torch.Generator(device=DEV).manual_seed(5)
